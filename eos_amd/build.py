@@ -32,6 +32,7 @@ ARCH = "gfx950"
 # (code object symbol stem, device source)
 DEVICE_SOURCES = [
     ("tq", os.path.join(CSRC, "kernels", "tq_kernels.hip")),
+    ("tqe", os.path.join(CSRC, "kernels", "tqe_kernels.hip")),
     ("enc", os.path.join(CSRC, "kernels", "enc_kernels.hip")),
     ("ret", os.path.join(CSRC, "kernels", "ret_kernels.hip")),
 ]

@@ -23,6 +23,8 @@ extern "C" {
 // Code objects built offline for gfx950 and linked in by eoship_blobs.S.
 extern const unsigned char eoship_tq_co_begin[];
 extern const unsigned char eoship_tq_co_end[];
+extern const unsigned char eoship_tqe_co_begin[];
+extern const unsigned char eoship_tqe_co_end[];
 extern const unsigned char eoship_enc_co_begin[];
 extern const unsigned char eoship_enc_co_end[];
 extern const unsigned char eoship_ret_co_begin[];
@@ -61,6 +63,9 @@ int Runtime::function(const char* name, hipFunction_t* out, char** err) {
   for (hipModule_t m : builtin) {
     e = hipModuleGetFunction(&f, m, name);
     if (e == hipSuccess) break;
+    // Not in this code object: take the error back, or the host program's
+    // next error check would report it.
+    (void)hipGetLastError();
   }
   if (e != hipSuccess) return hip_err(err, name, e);
   fns.emplace(name, f);
@@ -223,7 +228,8 @@ int eoship_runtime_create(int device, EosHipRuntime** out, char** err) {
     delete rt;
     return hip_err(err, "hipStreamCreateWithFlags", e);
   }
-  const unsigned char* images[3][2] = {{eoship_tq_co_begin, eoship_tq_co_end},
+  const unsigned char* images[4][2] = {{eoship_tq_co_begin, eoship_tq_co_end},
+                                       {eoship_tqe_co_begin, eoship_tqe_co_end},
                                        {eoship_enc_co_begin, eoship_enc_co_end},
                                        {eoship_ret_co_begin, eoship_ret_co_end}};
   for (auto& im : images) {

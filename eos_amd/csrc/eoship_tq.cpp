@@ -128,6 +128,12 @@ struct EosHipTQ {
   void* packed = nullptr;
   float* norms = nullptr;
   float* rot_t = nullptr;
+  // Encoding: R row-major and its split operand fragments (rot_frag NULL: no
+  // rotation, or scales outside the split product's bound), the largest row
+  // norm of R and the decision distance in half level steps.
+  float* rot_r = nullptr;
+  void* rot_frag = nullptr;
+  float rot_rmax = 0.f, enc_delta2 = 0.f;
   double* qrot = nullptr;  // [kMaxCols][d] rotated query columns
   // per-batch device scratch
   int8_t* bfrag = nullptr;
@@ -179,8 +185,8 @@ struct EosHipTQ {
   // reported in its place. Empty / nullptr for index order.
   long long* id_map = nullptr;
   std::vector<int64_t> rank_host;
-  // Handles sharing the corpus arrays (packed, norms, rot_t, tile_cn,
-  // codes_rm, id_map) through eoship_tq_share; nullptr while this is the only one.
+  // Handles sharing the corpus arrays (packed, norms, rot_t, rot_r, rot_frag,
+  // tile_cn, codes_rm, id_map) through eoship_tq_share; nullptr while this is the only one.
   int* corpus_refs = nullptr;
 
   void free_all() {
@@ -192,7 +198,7 @@ struct EosHipTQ {
     if (corpus_refs != nullptr && --*corpus_refs > 0) return;
     delete corpus_refs;
     corpus_refs = nullptr;
-    void* corpus[] = {packed, norms, rot_t, tile_cn, codes_rm, id_map};
+    void* corpus[] = {packed, norms, rot_t, rot_r, rot_frag, tile_cn, codes_rm, id_map};
     for (void* p : corpus)
       if (p) hipFree(p);
   }
@@ -215,6 +221,65 @@ struct EosHipTQ {
                   reinterpret_cast<void**>(&samp), err) != 0)
       return 1;
     return 0;
+  }
+
+  // 32-coordinate tiles and 32-wide K chunks (an even number) of the encode's
+  // split product.
+  int enc_tiles() const { return (d + 31) / 32; }
+  int enc_chunks() const { return (d + 63) / 64 * 2; }
+
+  // The rotation's operands of eos_tq_encode_split_* and the bound that
+  // gives its decision distance: with R = Rh + Rl + Re and x = xh + xl + xe in
+  // bf16 pairs, |u~ - u| / |x| <=
+  //   |R_j| 2^-18 + max|Re_j| + max|Rl_j| 2^-9     (R xe, Re x, Rl xl dropped)
+  // + |R_j| 33 * 2^-23     (32 products of a chunk summed in f32, an ulp lost
+  //                         at each addition whatever the order)
+  // + |R_j| chunks * 2^-24 (the sum over the chunks)
+  // with 5 % on top for the second-order terms (d = 384: 1.1e-5). Scales that
+  // would put the distance over a quarter of a half step, or leave f32 and
+  // bf16 no room, keep the f64 kernels (rot_frag stays NULL).
+  int prepare_encode(const float* rot, char** err) {
+    auto bf16 = [](float v) {  // round to nearest even
+      uint32_t u;
+      memcpy(&u, &v, 4);
+      u = (u + 0x7fffu + ((u >> 16) & 1u)) & 0xffff0000u;
+      memcpy(&v, &u, 4);
+      return v;
+    };
+    double rmax = 0.0, lmax = 0.0, emax = 0.0;
+    bool finite = true;
+    for (int j = 0; j < d; ++j) {
+      double ss = 0.0, sl = 0.0, se = 0.0;
+      for (int k = 0; k < d; ++k) {
+        const float v = rot[(size_t)j * d + k];
+        const float rest = v - bf16(v), low = bf16(rest), left = rest - low;
+        ss += (double)v * v;
+        sl += (double)low * low;
+        se += (double)left * left;
+      }
+      finite = finite && std::isfinite(ss);
+      rmax = std::max(rmax, ss);
+      lmax = std::max(lmax, sl);
+      emax = std::max(emax, se);
+    }
+    rmax = std::sqrt(rmax) * (1.0 + 1e-6);
+    const double bound = 1.05 * (rmax * (0x1p-18 + 33 * 0x1p-23 + enc_chunks() * 0x1p-24) +
+                                 std::sqrt(emax) + std::sqrt(lmax) * 0x1p-9);
+    const double delta2 = 2.0 * bound / (double)cb_scale + 1e-4;
+    if (!finite || !(rmax >= 0x1p-20 && rmax <= 0x1p20) || !(cb_scale <= 0x1p20f) || !(delta2 < 0.25))
+      return 0;
+    rot_rmax = (float)(rmax * (1.0 + 1e-6));
+    enc_delta2 = (float)(delta2 * (1.0 + 1e-6));
+    const size_t bytes = (size_t)d * d * sizeof(float);
+    if (rt->alloc(bytes, reinterpret_cast<void**>(&rot_r), err) != 0) return 1;
+    hipError_t e = rt->copy_sync(rot_r, rot, bytes, hipMemcpyHostToDevice);
+    if (e != hipSuccess) return hip_err(err, "hipMemcpy(rotation rows)", e);
+    if (rt->alloc((size_t)enc_tiles() * enc_chunks() * 4096, &rot_frag, err) != 0) return 1;
+    TqRotFragArgs f{rot_r, rot_frag, d, enc_tiles(), enc_chunks()};
+    const unsigned threads = (unsigned)(f.jtiles * f.nchunk) * 128u;
+    if (rt->launch("eos_tq_rot_frag", dim3((threads + 255) / 256), dim3(256), 0, &f, err) != 0)
+      return 1;
+    return rt->sync(err);
   }
 
   int ensure(void** p, size_t* have, size_t need, char** err) {
@@ -787,6 +852,7 @@ int eoship_tq_bind_corpus_opts(EosHipRuntime* rt, const EosHipTQDesc* desc, cons
       hip_err(err, "hipMemcpy(rotation)", e);
       return fail();
     }
+    if (tq->prepare_encode(desc->rotation, err) != 0) return fail();
   }
   if (!map_host.empty()) {
     if (rt->alloc(map_host.size() * sizeof(long long), reinterpret_cast<void**>(&tq->id_map), err) != 0)
@@ -854,6 +920,10 @@ int eoship_tq_share(EosHipRuntime* rt, EosHipTQ* src, EosHipTQ** out, char** err
   tq->packed = src->packed;
   tq->norms = src->norms;
   tq->rot_t = src->rot_t;
+  tq->rot_r = src->rot_r;
+  tq->rot_frag = src->rot_frag;
+  tq->rot_rmax = src->rot_rmax;
+  tq->enc_delta2 = src->enc_delta2;
   tq->tile_cn = src->tile_cn;
   tq->codes_rm = src->codes_rm;
   tq->id_map = src->id_map;
@@ -1603,9 +1673,66 @@ int eoship_tq_parent_topk(EosHipRuntime* rt, EosHipTQParents* parents, const flo
 
 namespace {
 
+// Rotated encodes on the matrix cores (see eos_tq_encode_split_*).
+int encode_split(EosHipRuntime* rt, EosHipTQ* tq, const float* d_x, int64_t n, uint8_t* d_codes,
+                 float* d_norms, char** err) {
+  constexpr int kRows = 96;  // vectors per workgroup
+  TqEncSplitArgs a;
+  memset(&a, 0, sizeof(a));
+  a.rot_r = tq->rot_r;
+  a.rfrag = tq->rot_frag;
+  a.d = tq->d;
+  a.bits = tq->bits;
+  a.row_bytes = tq->row_bytes;
+  a.nchunk = tq->enc_chunks();
+  a.jtiles = tq->enc_tiles();
+  a.cb_scale = tq->cb_scale;
+  a.delta2 = tq->enc_delta2;
+  a.rmax = tq->rot_rmax;
+  const bool vec = tq->d % 4 == 0 && (reinterpret_cast<uintptr_t>(d_x) & 15) == 0;
+  a.words = tq->row_bytes % 4 == 0 && (reinterpret_cast<uintptr_t>(d_codes) & 3) == 0 ? 1 : 0;
+  const int levels = 1 << tq->bits;
+  for (int v = 0; v < levels; ++v) a.cb[v] = tq->codebook[v];
+  // Distinct levels ascending, each with the first code that has it (ties go
+  // to the lower code).
+  std::vector<std::pair<int, int>> lv;
+  for (int v = 0; v < levels; ++v) lv.emplace_back(a.cb[v], v);
+  std::sort(lv.begin(), lv.end());
+  for (const auto& l : lv) {
+    if (a.m > 0 && a.lv[a.m - 1] == l.first) continue;
+    a.lv[a.m] = l.first;
+    a.li[a.m++] = l.second;
+  }
+  // The fewest workgroups side by side that 12 multiplying wavefronts (32
+  // coordinates each) cover, and the smallest of 4, 8, 12 that then do: each
+  // workgroup side by side splits the same vectors again (d = 384, 10^6
+  // vectors: 12 wavefronts 1.35 ms, 2 x 8 1.88, 3 x 4 1.55; d = 768, 300,000:
+  // 2 x 12 1.38 ms, 3 x 8 1.54), and wavefronts without coordinates idle
+  // (d = 128: 4 wavefronts 0.29 ms, 8 0.43).
+  a.jblocks = (a.jtiles + 11) / 12;
+  const int per = (a.jtiles + a.jblocks - 1) / a.jblocks;
+  const int nw = per <= 4 ? 4 : per <= 8 ? 8 : 12;
+  char name[40];
+  snprintf(name, sizeof(name), "eos_tq_encode_split_w%d%s", nw, vec ? "_v" : "");
+  // At most 2^24 vectors per launch (grid size).
+  const int64_t step = (int64_t)1 << 24;
+  for (int64_t i0 = 0; i0 < n; i0 += step) {
+    a.n = std::min(step, n - i0);
+    a.x = d_x + (size_t)i0 * tq->d;
+    a.codes = d_codes + (size_t)i0 * tq->row_bytes;
+    a.norms = d_norms + i0;
+    const int64_t vblocks = ((a.n + kRows - 1) / kRows + 7) / 8 * 8;
+    if (rt->launch(name, dim3((unsigned)(vblocks * a.jblocks)), dim3(64 * (nw + 4)), 0, &a, err,
+                   "tq_encode") != 0)
+      return 1;
+  }
+  return 0;
+}
+
 int encode_impl(EosHipRuntime* rt, EosHipTQ* tq, const float* d_x, int64_t n, uint8_t* d_codes,
                 float* d_norms, char** err) {
   if (n == 0) return 0;
+  if (tq->rot_frag != nullptr) return encode_split(rt, tq, d_x, n, d_codes, d_norms, err);
   TqEncodeArgs a;
   memset(&a, 0, sizeof(a));
   a.rot_t = tq->rot_t;

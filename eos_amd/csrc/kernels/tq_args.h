@@ -195,6 +195,33 @@ struct TqEncodeArgs {
   int cb[16];
 };
 
+// Rotation as the split product's operand fragments (eos_tq_rot_frag).
+struct TqRotFragArgs {
+  const float* rot_r;      // [d][d] R, row-major
+  void* frag;              // [jtiles][nchunk][2][2][64][16 bytes]
+  int d, jtiles, nchunk;   // 32-coordinate tiles; 32-wide K chunks (even)
+};
+
+// Encode with the rotation as a split bf16 product (eos_tq_encode_split_*).
+struct TqEncSplitArgs {
+  const float* x;          // [n][d]
+  const float* rot_r;      // [d][d] R, row-major
+  const void* rfrag;       // eos_tq_rot_frag's output
+  uint8_t* codes;          // [n][row_bytes]
+  float* norms;            // [n]
+  long long n;
+  int d, bits, row_bytes;
+  int nchunk, jtiles;      // as TqRotFragArgs
+  int jblocks;             // workgroups side by side over the coordinates
+  float cb_scale;
+  float delta2;            // decision distance in half level steps
+  float rmax;              // >= the largest row norm of R
+  int words;               // code rows are 4-byte aligned
+  int m;                   // distinct levels
+  int lv[16], li[16];      // the distinct levels ascending, and the first code of each
+  int cb[16];
+};
+
 // Inner-product layout (MSE codes + QJL signs + ResNorm + Norm): encode,
 // query preparation and exhaustive scores.
 struct TqIpArgs {

@@ -1,0 +1,485 @@
+// TurboQuant corpus encoders on gfx950: f32 vectors -> codes and norms, with
+// the rotation (and the residual sketch) on the matrix cores.
+//
+// The contract is the f64 one of eos_tq_encode_* (tq_kernels.hip): u_j one
+// fma chain over k, norm from the f64 chain of x^2, code_j the first level
+// nearest u_j. eos_tq_encode_split reaches the same codes and norms from
+// bounded approximations and decides in f64 only what the bound leaves open.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "tq_args.h"
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef double v4d __attribute__((ext_vector_type(4)));
+
+#define EOS_DEV __device__ __forceinline__
+
+namespace {
+
+EOS_DEV uint32_t bf16_bits(float v) { return __builtin_bit_cast(uint16_t, (__bf16)v); }
+EOS_DEV float bf16_val(uint32_t b) { return __uint_as_float(b << 16); }
+
+// Barrier for LDS data only: global loads in flight stay in flight.
+EOS_DEV void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+}  // namespace
+
+// R (row-major) as the split product's first operand: per 32 coordinates jt
+// and 32-wide K chunk, [K step of 16][high, low][lane][8 bf16], lane l holding
+// row 32 jt + l % 32 and K values 16 step + 8 (l / 32) .. + 7; zero past d.
+// high = bf16(R), low = bf16(R - high). One thread per 8 values.
+extern "C" __global__ __launch_bounds__(256) void eos_tq_rot_frag(TqRotFragArgs a) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= a.jtiles * a.nchunk * 2 * 64) return;
+  const int lane = i & 63, ks = (i >> 6) & 1, jc = i >> 7;
+  const int c = jc % a.nchunk, jt = jc / a.nchunk;
+  const int j = 32 * jt + (lane & 31), k0 = 32 * c + 16 * ks + 8 * (lane >> 5);
+  uint32_t h[8], lo[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float v = (j < a.d && k0 + e < a.d) ? a.rot_r[(size_t)j * a.d + k0 + e] : 0.0f;
+    h[e] = bf16_bits(v);
+    lo[e] = bf16_bits(v - bf16_val(h[e]));
+  }
+  v4i* out = reinterpret_cast<v4i*>(a.frag) + (size_t)(jc * 2 + ks) * 128 + lane;
+  v4i hv, lv;
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    hv[p] = (int)(h[2 * p] | (h[2 * p + 1] << 16));
+    lv[p] = (int)(lo[2 * p] | (lo[2 * p + 1] << 16));
+  }
+  out[0] = hv;
+  out[64] = lv;
+}
+
+namespace {
+
+constexpr int kSplitRows = 96;     // vectors per workgroup
+constexpr int kSplitItems = 1024;  // undecided (vector, coordinate) pairs listed per workgroup
+constexpr int kSplitStage = 4;     // staging wavefronts
+
+// Workgroup: 96 vectors x 32 NW coordinates, wavefront w < NW the coordinates
+// [32 w, + 32). K advances in chunks of 32 through two LDS stages; each staged
+// f32 value becomes a bf16 pair high + low, and
+//   u~ = sum over chunks of (Rh xl + Rl xh + Rh xh)
+// on bf16 MFMA, every chunk into a fresh accumulator that is then added in
+// f32. The host's bound E on |u~ - u| / |x| (prepare_encode) covers the split,
+// the 32 large products of a chunk summed in f32 in any order and the sum over
+// the chunks. In half steps of the integer level grid, w = 2 u~ / (nrm s_c),
+// the decision points are whole numbers (sums of neighbouring levels): a
+// 512-entry table indexed by the nearest whole number gives the codes on its
+// two sides and whether it is a decision point. Values closer to one than
+// delta2 = 2 E / s_c (+ 1e-4 for the rounding of w) go to a list and are
+// decided in f64: first from a sum in another order with its own bound, then,
+// if that is not enough (exact ties), by the contract's fma chain. The list
+// holds about 1 of 600 coordinates at d = 384, 4 bits; when it overflows every
+// pair of the workgroup is decided that way.
+// The norm's f64 sum is taken in another order too: it is kept when the f32
+// norms of its two error bounds agree, else recomputed as the chain.
+// A vector of norm 0 has u = 0 and every distance 0, one of infinite or NaN
+// norm no finite distance: both take code 0. Norms outside [2^-90, 2^100]
+// leave every coordinate to the list (bf16 over- and underflow).
+//
+// Bound: 10^6 x 384, 4 bits: 1.35-1.43 ms (the f64 kernel 27.3 ms, 14 % of
+// the f64 rate), of which the chunk loop takes about 0.83 ms (0.88 PFLOP of
+// bf16 products, 1.06 PFLOP/s), the listed pairs 0.14 ms and the start, norms,
+// decisions and stores of a workgroup the rest; the vectors read at 1.2 TB/s.
+// 96 rows keep R's fragments (590 KB per workgroup from L2) at 9 MFMAs a KB
+// within the 128 registers of four wavefronts per SIMD. Workgroups that stay
+// for many tiles, with the list left to the staging wavefronts, measured
+// slower (1.58 ms: those four then pace the chunks), as did splitting by the
+// multiplying wavefronts themselves (1.44).
+//
+// Wavefronts [0, NW) multiply and decide; the other four stage: while a chunk
+// is multiplied out of one LDS stage they split the next into the other, with
+// the two after it in flight. One barrier per chunk, at which both sides meet;
+// then all wavefronts decide the listed pairs and write the codes.
+template <int NW, bool VEC>
+struct EncodeSplit {
+  static constexpr int PT = 64 * kSplitStage;   // staging threads
+  static constexpr int NT = 64 * NW + PT;
+  static constexpr int BM = kSplitRows, RT = BM / 32;
+  static constexpr int U = BM * 8 / PT;         // 16-byte loads per staging thread per chunk
+  static_assert(BM * 8 % PT == 0, "staging split");
+  static constexpr int CST = NW * 16 + 4;       // code bytes per vector (4 bits), padded
+  struct Lds {
+    uint32_t xs[2][2][BM * 16];
+    uint8_t cbuf[BM * CST];
+    double s64[BM];
+    float inv2[BM], dlim[BM];
+    uint32_t items[kSplitItems];
+    uint32_t nitems;
+    uint16_t lut[512];
+  };
+  const TqEncSplitArgs& a;
+  Lds& s;
+  // The tile: nv vectors from v0 on, 32-coordinate tiles from jt0 on.
+  long long v0;
+  int nv, jt0;
+
+  EOS_DEV void multiply(int wave, int lane) {
+    const int g = lane >> 5, l32 = lane & 31, d = a.d;
+    const bool active = jt0 + wave < a.jtiles;
+    const v4i* src = reinterpret_cast<const v4i*>(a.rfrag) +
+                     (size_t)min(jt0 + wave, a.jtiles - 1) * a.nchunk * 256 + lane;
+    auto load_r = [&](v4i (&rf)[4], int c) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) rf[i] = src[(size_t)c * 256 + 64 * i];
+    };
+    v16f tot[RT];
+    auto compute = [&](int st, const v4i (&rf)[4]) {
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+        // The cross products first: the accumulator is small while they add.
+        v16f acc = v16f{0};
+        v8bf bh[2];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+          const int o = (32 * rt + l32) * 16 + ((2 * ks + g) ^ ((l32 >> 2) & 3)) * 4;
+          bh[ks] = __builtin_bit_cast(v8bf, *reinterpret_cast<const v4i*>(&s.xs[st][0][o]));
+          const v8bf bl = __builtin_bit_cast(v8bf, *reinterpret_cast<const v4i*>(&s.xs[st][1][o]));
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, rf[2 * ks]), bl, acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, rf[2 * ks + 1]), bh[ks], acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, rf[2 * ks]), bh[ks], acc, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) tot[rt][i] += acc[i];
+      }
+    };
+    v4i rfa[4], rfb[4];
+    load_r(rfa, 0);
+    // The decision table: cell c = nearest whole number of w, [-256, 255].
+    for (int i = 64 * wave + lane; i < 512; i += 64 * NW) {
+      const int c = i - 256;
+      int below = 0, upto = 0;
+      for (int l = 0; l + 1 < a.m; ++l) {
+        const int p = a.lv[l] + a.lv[l + 1];
+        below += p < c ? 1 : 0;
+        upto += p <= c ? 1 : 0;
+      }
+      s.lut[i] = (uint16_t)(a.li[below] | (a.li[upto] << 4) | (upto != below ? 0x1000 : 0));
+    }
+    if (wave == 0 && lane == 0) s.nitems = 0u;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) tot[rt] = v16f{0};
+    lds_barrier();
+    for (int c = 0; c < a.nchunk; c += 2) {
+      load_r(rfb, c + 1);
+      if (active) compute(0, rfa);
+      lds_barrier();
+      load_r(rfa, min(c + 2, a.nchunk - 1));
+      if (active) compute(1, rfb);
+      lds_barrier();
+    }
+    // Codes of the wavefront's 32 coordinates: element 4 q + e of a lane
+    // is coordinate 8 q + 4 g + e of vector 32 rt + l32.
+    if (active) {
+      const int left = d - 32 * (jt0 + wave);  // coordinates from the wavefront's first
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+        const int v = 32 * rt + l32;
+        const float iv = s.inv2[v], dl = s.dlim[v];
+        const uint32_t keep = dl < -1.0f ? 0u : 0xffffu;
+        const uint32_t force = dl > 1.0f ? 0xf000u : 0u;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          uint32_t pk = 0, fl = force;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            // c = w to the nearest whole number, through the low mantissa
+            // bits of w + 1.5 * 2^23, clamped to the table; r = w - c.
+            constexpr float kM = 12582912.0f;
+            const float x = tot[rt][4 * q + e];
+            const float f = __builtin_amdgcn_fmed3f(__builtin_fmaf(x, iv, kM), kM - 256.0f, kM + 255.0f);
+            const float r = __builtin_fmaf(x, iv, kM - f);
+            const uint32_t ent = s.lut[__float_as_uint(f) - (0x4b400000u - 256u)];
+            pk |= ((ent >> (r > 0.0f ? 4 : 0)) & 15u) << (e * a.bits);
+            fl |= (fabsf(r) > dl ? 0u : ent) << e;
+          }
+          pk &= keep;
+          fl &= 0xf000u;
+          const int valid = left - (8 * q + 4 * g);
+          if (left < 32 && valid < 4) {
+            const int m = valid < 0 ? 0 : valid;
+            pk &= (1u << (m * a.bits)) - 1u;
+            fl &= ((1u << m) - 1u) << 12;
+          }
+          if (fl != 0u) {
+#pragma unroll 1
+            for (fl >>= 12; fl != 0u; fl &= fl - 1u) {
+              const uint32_t pos = atomicAdd(&s.nitems, 1u);
+              if (pos < (uint32_t)kSplitItems)
+                s.items[pos] =
+                    (uint32_t)v << 16 | (uint32_t)(32 * wave + 8 * q + 4 * g + (__ffs(fl) - 1));
+            }
+          }
+          if (a.bits == 4)
+            *reinterpret_cast<uint16_t*>(&s.cbuf[v * CST + wave * 16 + 4 * q + 2 * g]) = (uint16_t)pk;
+          else
+            s.cbuf[v * CST + wave * 8 + 2 * q + g] = (uint8_t)pk;
+        }
+      }
+    }
+  }
+
+  // Pair i of the list (or of the whole tile) by 16 lanes: every lane's
+  // 16-byte pieces of the two rows are requested six at a time.
+  EOS_DEV void decide(int i, bool all, int jn, int sub) {
+    const int d = a.d;
+    const int v = all ? i / jn : (int)(s.items[i] >> 16);
+    const int jl = all ? i - v * jn : (int)(s.items[i] & 0xffffu);
+    if (s.dlim[v] < -1.0f) return;
+    const float* xv = a.x + (size_t)(v0 + v) * d;
+    const float* rj = a.rot_r + (size_t)(32 * jt0 + jl) * d;
+    double u = 0.0;
+    if constexpr (VEC) {
+      for (int k0 = 4 * sub; k0 < d; k0 += 384) {
+        float4 xk[6], rk[6];
+#pragma unroll
+        for (int p = 0; p < 6; ++p) {
+          const int k = min(k0 + 64 * p, d - 4);
+          xk[p] = *reinterpret_cast<const float4*>(xv + k);
+          rk[p] = *reinterpret_cast<const float4*>(rj + k);
+        }
+#pragma unroll
+        for (int p = 0; p < 6; ++p) {
+          double w = (double)rk[p].x * (double)xk[p].x;
+          w = fma((double)rk[p].y, (double)xk[p].y, w);
+          w = fma((double)rk[p].z, (double)xk[p].z, w);
+          w = fma((double)rk[p].w, (double)xk[p].w, w);
+          u += k0 + 64 * p < d ? w : 0.0;
+        }
+      }
+    } else {
+      for (int k0 = sub; k0 < d; k0 += 192) {
+        float xk[12], rk[12];
+#pragma unroll
+        for (int p = 0; p < 12; ++p) {
+          const int k = min(k0 + 16 * p, d - 1);
+          xk[p] = xv[k];
+          rk[p] = rj[k];
+        }
+#pragma unroll
+        for (int p = 0; p < 12; ++p)
+          u = fma(k0 + 16 * p < d ? (double)rk[p] : 0.0, (double)xk[p], u);
+      }
+    }
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) u += __shfl_xor(u, o);
+    if (sub != 0) return;
+    const double nrm = __builtin_sqrt(s.s64[v]);
+    double d1 = __builtin_inf(), d2 = __builtin_inf();
+    int code = 0;
+#pragma unroll 1
+    for (int l = 0; l < a.m; ++l) {
+      const double dv = fabs(u - nrm * ((double)a.cb_scale * (double)a.lv[l]));
+      if (dv < d1) {
+        d2 = d1;
+        d1 = dv;
+        code = a.li[l];
+      } else if (dv < d2) {
+        d2 = dv;
+      }
+    }
+    const double err = (4.0 * d + 32.0) * 2.220446049250313e-16 * nrm *
+                       ((double)a.rmax + 128.0 * (double)a.cb_scale);
+    if (!(d2 - d1 > 2.0 * err)) {
+      // The contract's own chain.
+      double ue = 0.0, se = 0.0;
+#pragma unroll 1
+      for (int k = 0; k < d; ++k) {
+        ue = fma((double)rj[k], (double)xv[k], ue);
+        se = fma((double)xv[k], (double)xv[k], se);
+      }
+      const double ne = __builtin_sqrt(se);
+      double bd = 0.0;
+      code = 0;
+#pragma unroll 1
+      for (int l = 0; l < (1 << a.bits); ++l) {
+        const double dv = fabs(ue - ne * ((double)a.cb_scale * (double)a.cb[l]));
+        if (l == 0 || dv < bd) {
+          bd = dv;
+          code = l;
+        }
+      }
+    }
+    const int bit = jl * a.bits;
+    const int off = v * CST + (bit >> 3), sh = (off & 3) * 8 + (bit & 7);
+    uint32_t* word = reinterpret_cast<uint32_t*>(&s.cbuf[off & ~3]);
+    atomicAnd(word, ~(((1u << a.bits) - 1u) << sh));
+    atomicOr(word, (uint32_t)code << sh);
+  }
+
+  // Code rows: the tile's bytes of each vector.
+  EOS_DEV void write(int tid) {
+    const int rb0 = 4 * jt0 * a.bits;
+    const int nb = min(a.row_bytes - rb0, 4 * NW * a.bits);
+    uint8_t* out = a.codes + (size_t)v0 * a.row_bytes + rb0;
+    if (a.words) {
+      const int nw = nb >> 2;
+      for (int i = tid; i < nv * nw; i += NT) {
+        const int v = i / nw, b = i - v * nw;
+        *reinterpret_cast<uint32_t*>(out + (size_t)v * a.row_bytes + 4 * b) =
+            *reinterpret_cast<const uint32_t*>(&s.cbuf[v * CST + 4 * b]);
+      }
+    } else {
+      for (int i = tid; i < nv * nb; i += NT) {
+        const int v = i / nb, b = i - v * nb;
+        out[(size_t)v * a.row_bytes + b] = s.cbuf[v * CST + b];
+      }
+    }
+  }
+
+  EOS_DEV void stage(int tid) {
+    const int d = a.d;
+    // Thread t stages 4 values (16 bytes) of rows t / 8 + u PT / 8 per chunk.
+    // Loads come from clamped positions; what lies past d or n is cleared
+    // when the values are stored, so that no load is waited for before that.
+    const int slot = tid & 7, row0 = tid >> 3;
+    auto load = [&](float (&xr)[U][4], int c) {
+      const int k = 32 * c + 4 * slot;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float* src = a.x + (size_t)min(v0 + row0 + u * (PT / 8), a.n - 1) * d;
+        if constexpr (VEC) {
+          const float4 v = *reinterpret_cast<const float4*>(src + min(k, d - 4));
+          xr[u][0] = v.x;
+          xr[u][1] = v.y;
+          xr[u][2] = v.z;
+          xr[u][3] = v.w;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) xr[u][e] = src[min(k + e, d - 1)];
+        }
+      }
+    };
+    double ss[U];
+    // Row r's 64 bytes of a stage are four 16-byte groups of 8 K values; group
+    // q sits at q ^ ((r >> 2) & 3), so that a fragment read covers all banks.
+    auto store = [&](const float (&xr)[U][4], int st, int c) {
+      const int k = 32 * c + 4 * slot;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int r = row0 + u * (PT / 8);
+        uint32_t h[4], lo[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float v = (r < nv && k + (VEC ? 0 : e) < d) ? xr[u][e] : 0.0f;
+          ss[u] = fma((double)v, (double)v, ss[u]);
+          h[e] = bf16_bits(v);
+          lo[e] = bf16_bits(v - bf16_val(h[e]));
+        }
+        const int o = r * 16 + (((slot >> 1) ^ ((r >> 2) & 3)) * 4) + (slot & 1) * 2;
+        *reinterpret_cast<uint2*>(&s.xs[st][0][o]) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+        *reinterpret_cast<uint2*>(&s.xs[st][1][o]) = make_uint2(lo[0] | (lo[1] << 16), lo[2] | (lo[3] << 16));
+      }
+    };
+    // Norms, and each vector's scale of w and decision distance.
+    auto norms = [&](bool out) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        double sq = ss[u];
+        sq += __shfl_xor(sq, 1);
+        sq += __shfl_xor(sq, 2);
+        sq += __shfl_xor(sq, 4);
+        const int r = row0 + u * (PT / 8);
+        if (slot != 0) continue;
+        const double nrm = __builtin_sqrt(sq);
+        if (out && r < nv) {
+          const double eps = (double)(d + 8) * 2.220446049250313e-16;
+          float nf = (float)nrm;
+          if (!((float)__builtin_sqrt(sq * (1.0 - eps)) == (float)__builtin_sqrt(sq * (1.0 + eps)))) {
+            const float* src = a.x + (size_t)(v0 + r) * d;
+            double w = 0.0;
+#pragma unroll 1
+            for (int k = 0; k < d; ++k) w = fma((double)src[k], (double)src[k], w);
+            nf = (float)__builtin_sqrt(w);
+          }
+          a.norms[v0 + r] = nf;
+        }
+        float iv = 0.0f, dl = -2.0f;  // code 0 throughout
+        if (nrm > 0.0 && nrm < __builtin_inf()) {
+          if (nrm >= 0x1p-90 && nrm <= 0x1p100) {
+            iv = (float)(2.0 / (nrm * (double)a.cb_scale));
+            dl = a.delta2;
+          } else {
+            dl = __builtin_inff();  // every coordinate to the list
+          }
+        }
+        s.s64[r] = sq;
+        s.inv2[r] = iv;
+        s.dlim[r] = dl;
+      }
+    };
+#pragma unroll
+    for (int u = 0; u < U; ++u) ss[u] = 0.0;
+    float xa[U][4], xb[U][4];
+    load(xa, 0);
+    load(xb, 1);
+    store(xa, 0, 0);
+    load(xa, 2);
+    lds_barrier();
+    for (int c = 0; c + 2 < a.nchunk; c += 2) {
+      store(xb, 1, c + 1);
+      load(xb, c + 3);
+      lds_barrier();
+      store(xa, 0, c + 2);
+      load(xa, c + 4);
+      lds_barrier();
+    }
+    store(xb, 1, a.nchunk - 1);
+    lds_barrier();
+    norms(jt0 == 0);  // while the last chunk is multiplied out
+    lds_barrier();
+  }
+
+  EOS_DEV void run() {
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // Workgroup w runs on XCD w % 8: the coordinate blocks of a vector block
+    // run back to back on one XCD, so its vectors are read into that L2 once.
+    const int l = blockIdx.x >> 3;
+    v0 = ((long long)(l / a.jblocks) * 8 + (blockIdx.x & 7)) * BM;
+    if (v0 >= a.n) return;
+    nv = (int)min((long long)BM, a.n - v0);
+    jt0 = l % a.jblocks * NW;
+    if (wave < NW)
+      multiply(wave, tid & 63);
+    else
+      stage(tid - 64 * NW);
+    lds_barrier();
+    const bool all = s.nitems > (uint32_t)kSplitItems;
+    const int jn = min(32 * NW, a.d - 32 * jt0);
+    const int total = all ? nv * jn : (int)s.nitems;
+#pragma unroll 1
+    for (int i = tid >> 4; i < total; i += NT / 16) decide(i, all, jn, tid & 15);
+    lds_barrier();
+    write(tid);
+  }
+};
+
+}  // namespace
+
+// NW multiplying wavefronts; x rows 16-byte aligned (_v) or not.
+#define EOS_TQ_ENCODE_SPLIT(NW)                                                            \
+  extern "C" __global__ __launch_bounds__(64 * (NW + kSplitStage)) __attribute__((amdgpu_waves_per_eu(4))) \
+  void eos_tq_encode_split_w##NW(TqEncSplitArgs a) {                                      \
+    __shared__ __attribute__((aligned(16))) EncodeSplit<NW, false>::Lds lds;              \
+    EncodeSplit<NW, false>{a, lds, 0, 0, 0}.run();                                              \
+  }                                                                                       \
+  extern "C" __global__ __launch_bounds__(64 * (NW + kSplitStage)) __attribute__((amdgpu_waves_per_eu(4))) \
+  void eos_tq_encode_split_w##NW##_v(TqEncSplitArgs a) {                                  \
+    __shared__ __attribute__((aligned(16))) EncodeSplit<NW, true>::Lds lds;               \
+    EncodeSplit<NW, true>{a, lds, 0, 0, 0}.run();                                               \
+  }
+EOS_TQ_ENCODE_SPLIT(4)
+EOS_TQ_ENCODE_SPLIT(8)
+EOS_TQ_ENCODE_SPLIT(12)
+#undef EOS_TQ_ENCODE_SPLIT
