@@ -1155,14 +1155,24 @@ int maxsim_check(EosHipRuntime* rt, EosHipTQ* tq, int32_t doc_len, int32_t q, in
   return 0;
 }
 
+// Chunks each of `rows` score rows of n splits into for its top kk: about one
+// workgroup per CU in all, at least 2048 (and 4 kk) elements each, lists that
+// eos_tq_finalize can merge.
+int rank_chunks(EosHipRuntime* rt, int rows, int64_t n, int kk) {
+  int64_t chunks = std::max<int64_t>(1, rt->compute_units / rows);
+  chunks = std::min<int64_t>(chunks, kSortCap / kk);
+  return (int)std::min<int64_t>(chunks, n / std::max<int64_t>(4 * (int64_t)kk, 2048));
+}
+
 // Top kk of each of `rows` score rows [rows][n] by (score desc, index asc)
 // into ids / scores [rows][kk]. With few rows, each row is split into
-// chunks so that about one workgroup per CU selects: every chunk's exact
-// top kk (keys unique, so exactly kk or the whole chunk), then
-// eos_tq_finalize merges each row's nchunks * kk keys; with many rows (or
+// rank_chunks: every chunk's exact top kk (keys unique, so exactly kk or the
+// whole chunk) into keys [rows][chunks * kk], then eos_tq_finalize merges
+// each row's (counts and status [rows] are its scratch); with many rows (or
 // a kk too large to merge) one workgroup ranks each row.
-int rank_rows(EosHipRuntime* rt, EosHipTQ* tq, const float* d_rows, int rows, int64_t n, int kk,
-              int64_t* d_ids, float* d_scores, char** err) {
+int rank_rows(EosHipRuntime* rt, const float* d_rows, int rows, int64_t n, int kk, int64_t* d_ids,
+              float* d_scores, unsigned long long* keys, uint32_t* counts, int* status,
+              const char* label, char** err) {
   TqSelectArgs sel;
   memset(&sel, 0, sizeof(sel));
   sel.rows = d_rows;
@@ -1172,38 +1182,28 @@ int rank_rows(EosHipRuntime* rt, EosHipTQ* tq, const float* d_rows, int rows, in
   sel.stride = n;
   sel.kk = kk;
   sel.nrows = rows;
-  int64_t chunks = std::max<int64_t>(1, rt->compute_units / rows);
-  chunks = std::min<int64_t>(chunks, kSortCap / kk);
-  chunks = std::min<int64_t>(chunks, n / std::max<int64_t>(4 * (int64_t)kk, 2048));
-  if (chunks <= 1) {
+  const int nch = rank_chunks(rt, rows, n, kk);
+  if (nch <= 1) {
     sel.mode = 1;
-    return rt->launch("eos_tq_row_select", dim3(rows), dim3(1024), 0, &sel, err,
-                      "tq_maxsim_select");
+    return rt->launch("eos_tq_row_select", dim3(rows), dim3(1024), 0, &sel, err, label);
   }
-  const int nch = (int)chunks;
-  if (tq->ensure(reinterpret_cast<void**>(&tq->sel_keys), &tq->sel_keys_bytes,
-                 (size_t)rows * nch * kk * sizeof(unsigned long long), err) != 0 ||
-      tq->ensure(reinterpret_cast<void**>(&tq->sel_aux), &tq->sel_aux_bytes,
-                 (size_t)rows * 2 * sizeof(uint32_t), err) != 0)
-    return 1;
   sel.mode = 2;
   sel.nchunks = nch;
-  sel.keys_out = tq->sel_keys;
-  sel.counts_out = tq->sel_aux;
-  if (rt->launch("eos_tq_row_select", dim3(rows, nch), dim3(1024), 0, &sel, err,
-                 "tq_maxsim_select") != 0)
+  sel.keys_out = keys;
+  sel.counts_out = counts;
+  if (rt->launch("eos_tq_row_select", dim3(rows, nch), dim3(1024), 0, &sel, err, label) != 0)
     return 1;
   TqFinalizeArgs f;
   memset(&f, 0, sizeof(f));
-  f.cand = tq->sel_keys;
-  f.cand_count = tq->sel_aux;
+  f.cand = keys;
+  f.cand_count = counts;
   f.ids = reinterpret_cast<long long*>(d_ids);
   f.scores = d_scores;
-  f.status = reinterpret_cast<int*>(tq->sel_aux + rows);
+  f.status = status;
   f.cap = nch * kk;
   f.kk = kk;
   f.q = rows;
-  return rt->launch(finalize_kernel(f.kk), dim3(rows), dim3(256), 0, &f, err, "tq_maxsim_select_merge");
+  return rt->launch(finalize_kernel(f.kk), dim3(rows), dim3(256), 0, &f, err, label);
 }
 
 // Bound-filtered MaxSim top-k of one prepared chunk of cq queries (kk <=
@@ -1379,8 +1379,14 @@ int maxsim_topk_impl(EosHipRuntime* rt, EosHipTQ* tq, int32_t doc_len, const flo
       if (tq->maxsim_pass(q0, qp, doc_len, 0, ndocs, tq->dense + (size_t)q0 * ndocs, err) != 0)
         return 1;
     }
-    if (rank_rows(rt, tq, tq->dense, cq, ndocs, kk, d_ids + (size_t)c0 * kk,
-                  d_scores + (size_t)c0 * kk, err) != 0)
+    const int nch = std::max(1, rank_chunks(rt, cq, ndocs, kk));
+    if (tq->ensure(reinterpret_cast<void**>(&tq->sel_keys), &tq->sel_keys_bytes,
+                   (size_t)cq * nch * kk * sizeof(unsigned long long), err) != 0 ||
+        tq->ensure(reinterpret_cast<void**>(&tq->sel_aux), &tq->sel_aux_bytes,
+                   (size_t)cq * 2 * sizeof(uint32_t), err) != 0 ||
+        rank_rows(rt, tq->dense, cq, ndocs, kk, d_ids + (size_t)c0 * kk,
+                  d_scores + (size_t)c0 * kk, tq->sel_keys, tq->sel_aux,
+                  reinterpret_cast<int*>(tq->sel_aux + cq), "tq_maxsim_select", err) != 0)
       return 1;
   }
   return 0;
@@ -1469,12 +1475,14 @@ struct EosHipTQParents {
   int64_t np = 0, live = 0;
   long long* off = nullptr;   // [np + 1]
   double* l1p = nullptr;      // [np] log1p(child count)
+  long long* long_ids = nullptr;  // [nlong] parents of more than EOS_PARENT_SHORT children
+  int64_t nlong = 0;
   float* pscores = nullptr;   // [per][np]
   size_t pscores_bytes = 0;
   void* io = nullptr;         // host-API staging
   size_t io_bytes = 0;
   ~EosHipTQParents() {
-    void* ptrs[] = {off, l1p, pscores, io};
+    void* ptrs[] = {off, l1p, long_ids, pscores, io};
     for (void* p : ptrs)
       if (p) hipFree(p);
   }
@@ -1526,24 +1534,26 @@ int parent_topk_impl(EosHipRuntime* rt, EosHipTQParents* P, const float* d_queri
     ag.l1p = P->l1p;
     ag.out = P->pscores;
     ag.np = P->np;
+    ag.out_stride = P->np;
     ag.stride = tq->n;
     ag.penalty = penalty;
     ag.top_n = top_n;
     ag.qb = qb;
-    if (rt->launch("eos_tq_parent_agg", dim3((unsigned)((P->np + 3) / 4), qb), dim3(256), 0, &ag,
-                   err, "tq_parent_agg") != 0)
+    // Short parents by a lane each, the others (listed at bind) by a wavefront.
+    if (P->nlong < P->np &&
+        rt->launch("eos_tq_parent_agg_short", dim3((unsigned)((P->np + 255) / 256), qb), dim3(256),
+                   0, &ag, err, "tq_parent_agg") != 0)
       return 1;
-    TqSelectArgs sel;
-    memset(&sel, 0, sizeof(sel));
-    sel.rows = P->pscores;
-    sel.ids = reinterpret_cast<long long*>(d_ids + (size_t)q0 * kk);
-    sel.scores = d_scores + (size_t)q0 * kk;
-    sel.n = P->np;
-    sel.stride = P->np;
-    sel.kk = kk;
-    sel.mode = 1;
-    sel.nrows = qb;
-    if (rt->launch("eos_tq_row_select", dim3(qb), dim3(1024), 0, &sel, err, "tq_parent_select") != 0)
+    if (P->nlong > 0) {
+      ag.np = P->nlong;
+      ag.list = P->long_ids;
+      if (rt->launch("eos_tq_parent_agg", dim3((unsigned)((P->nlong + 3) / 4), qb), dim3(256), 0,
+                     &ag, err, "tq_parent_agg") != 0)
+        return 1;
+    }
+    // The flat scan's candidate lists (kBatch x kCap keys) hold the chunks'.
+    if (rank_rows(rt, P->pscores, qb, P->np, kk, d_ids + (size_t)q0 * kk, d_scores + (size_t)q0 * kk,
+                  tq->cand, tq->cand_count, tq->status, "tq_parent_select", err) != 0)
       return 1;
     TqParentBestArgs bb;
     memset(&bb, 0, sizeof(bb));
@@ -1582,11 +1592,13 @@ int eoship_tq_parents_bind(EosHipRuntime* rt, EosHipTQ* tq, const int64_t* offse
     return set_err(err, "%s: offsets must start at 0 and end at the corpus size %lld", what,
                    (long long)tq->n);
   std::vector<double> l1p((size_t)nparents);
+  std::vector<long long> longs;
   int64_t live = 0;
   for (int64_t p = 0; p < nparents; ++p) {
     const int64_t c = offsets[p + 1] - offsets[p];
     if (c < 0) return set_err(err, "%s: offsets decrease at parent %lld", what, (long long)p);
     live += c > 0 ? 1 : 0;
+    if (c > EOS_PARENT_SHORT) longs.push_back((long long)p);
     l1p[(size_t)p] = std::log1p((double)c);
   }
   auto* P = new EosHipTQParents();
@@ -1596,12 +1608,16 @@ int eoship_tq_parents_bind(EosHipRuntime* rt, EosHipTQ* tq, const int64_t* offse
   const size_t ob = (size_t)(nparents + 1) * sizeof(long long), lb = (size_t)nparents * sizeof(double);
   hipError_t e = hipSuccess;
   if (rt->alloc(ob, reinterpret_cast<void**>(&P->off), err) ||
-      rt->alloc(lb, reinterpret_cast<void**>(&P->l1p), err)) {
+      rt->alloc(lb, reinterpret_cast<void**>(&P->l1p), err) ||
+      rt->alloc(longs.size() * sizeof(long long), reinterpret_cast<void**>(&P->long_ids), err)) {
     delete P;
     return 1;
   }
+  P->nlong = (int64_t)longs.size();
   e = rt->copy_sync(P->off, offsets, ob, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = rt->copy_sync(P->l1p, l1p.data(), lb, hipMemcpyHostToDevice);
+  if (e == hipSuccess && !longs.empty())
+    e = rt->copy_sync(P->long_ids, longs.data(), longs.size() * sizeof(long long), hipMemcpyHostToDevice);
   if (e != hipSuccess) {
     delete P;
     return hip_err(err, "hipMemcpy(parent offsets)", e);

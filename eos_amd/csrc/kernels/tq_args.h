@@ -133,6 +133,8 @@ struct TqMaxsimArgs {
 // [off[p], off[p+1]) of each score row; out[q][p] = f32(mean of its best
 // min(top_n, 5, count) child scores (f64 sum in descending order) -
 // penalty * l1p[p]); parents without children get -inf.
+// Children up to which one lane aggregates a parent (eos_tq_parent_agg_short).
+#define EOS_PARENT_SHORT 64
 struct TqParentArgs {
   const float* scores;      // [qb][stride] child scores
   const long long* off;     // [np + 1]
@@ -141,6 +143,10 @@ struct TqParentArgs {
   long long np, stride;
   double penalty;
   int top_n, qb;
+  // eos_tq_parent_agg: the parents it takes (np of them; p = list[i]), out
+  // rows out_stride apart; NULL: parent p = i.
+  const long long* list;
+  long long out_stride;
 };
 
 // Best child of each selected parent: the highest child score, ties to the
