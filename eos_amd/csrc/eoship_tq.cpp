@@ -2105,7 +2105,12 @@ int eoship_tq_ip_encode_device(EosHipRuntime* rt, const EosHipTQIPSpec* spec, co
   a.resnorms = d_resnorms;
   a.norms = d_norms;
   a.n = n;
-  return rt->launch("eos_tq_encode_ip", dim3((unsigned)((n + 7) / 8)), dim3(256), 0, &a, err,
+  // 128 coordinates per tile row of the kernel (TJ); 32 vectors per workgroup
+  // while their residuals fit the LDS beside the stages (d <= 512), else 16.
+  const int tj = (a.d + 127) / 128, per = tj <= 4 ? 32 : 16;
+  char name[32];
+  snprintf(name, sizeof(name), "eos_tq_encode_ip_t%d", tj);
+  return rt->launch(name, dim3((unsigned)((n + per - 1) / per)), dim3(512), 0, &a, err,
                     "tq_encode_ip");
 }
 

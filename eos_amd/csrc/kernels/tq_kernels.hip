@@ -477,110 +477,11 @@ extern "C" __global__ __launch_bounds__(256) void eos_tq_encode_d1024(TqEncodeAr
 // Build-defined inner-product layout after the published TurboQuant_prod
 // estimator (the quantizer is in the un-vendored module; byte layout of
 // runtime/turboquant_bytes.go:14-25): the MSE stage of encode_body, then a
-// 1-bit QJL sketch of the residual in the rotated frame, all in f64:
+// 1-bit QJL sketch of the residual in the rotated frame, all in f64
+// (encoded by eos_tq_encode_ip_t*):
 //   r_j = u_j - nrm c_code_j;  ResNorm = (float)(sqrt(sum_j r_j^2) / nrm)
 //   sign bit i = (sum_j S[i][j] r_j >= 0), fma chains in j order
-// Eight vectors per workgroup (d <= 1024); thread t runs coordinates and
-// sketch rows t, t + 256, ... for all eight, reading R^T and S^T coalesced.
-constexpr int kIpV = 8;
 constexpr int kIpDMax = 1024;
-extern "C" __global__ __launch_bounds__(256) void eos_tq_encode_ip(TqIpArgs a) {
-  __shared__ float xs[kIpDMax * kIpV];
-  __shared__ double rs[kIpV * kIpDMax];
-  __shared__ double ncs[kIpV * 16];
-  __shared__ uint8_t cs[kIpV * kIpDMax];
-  __shared__ uint8_t sb[kIpV * kIpDMax];
-  __shared__ double nrms[kIpV];
-  const int tid = threadIdx.x;
-  const long long v0 = (long long)blockIdx.x * kIpV;
-  const int nv = (int)min((long long)kIpV, a.n - v0);
-  if (nv <= 0) return;
-  const int d = a.d, levels = 1 << a.bits;
-  for (int i = tid; i < kIpV * d; i += 256) {
-    const int v = i / d, k = i - v * d;
-    xs[k * kIpV + v] = v < nv ? a.x[(size_t)(v0 + v) * d + k] : 0.0f;
-  }
-  __syncthreads();
-  if (tid < kIpV) {
-    double ss = 0.0;
-    for (int k = 0; k < d; ++k) {
-      const double xk = (double)xs[k * kIpV + tid];
-      ss = fma(xk, xk, ss);
-    }
-    const double nrm = __builtin_sqrt(ss);
-    nrms[tid] = nrm;
-    if (tid < nv) a.norms[v0 + tid] = (float)nrm;
-    for (int l = 0; l < levels; ++l) ncs[tid * 16 + l] = nrm * ((double)a.cb_scale * (double)a.cb[l]);
-  }
-  __syncthreads();
-  for (int j = tid; j < d; j += 256) {
-    double acc[kIpV];
-#pragma unroll
-    for (int v = 0; v < kIpV; ++v) acc[v] = a.rot_t != nullptr ? 0.0 : (double)xs[j * kIpV + v];
-    if (a.rot_t != nullptr) {
-      for (int k = 0; k < d; ++k) {
-        const double r = (double)a.rot_t[(size_t)k * d + j];
-#pragma unroll
-        for (int v = 0; v < kIpV; ++v) acc[v] = fma(r, (double)xs[k * kIpV + v], acc[v]);
-      }
-    }
-#pragma unroll
-    for (int v = 0; v < kIpV; ++v) {
-      const double u = acc[v];
-      int best = 0;
-      double bd = fabs(u - ncs[v * 16]);
-      for (int l = 1; l < levels; ++l) {
-        const double dv = fabs(u - ncs[v * 16 + l]);
-        if (dv < bd) {
-          bd = dv;
-          best = l;
-        }
-      }
-      cs[v * kIpDMax + j] = (uint8_t)best;
-      rs[v * kIpDMax + j] = u - ncs[v * 16 + best];
-    }
-  }
-  __syncthreads();
-  if (tid < nv) {
-    double rn = 0.0;
-    for (int j = 0; j < d; ++j) rn = fma(rs[tid * kIpDMax + j], rs[tid * kIpDMax + j], rn);
-    const double nrm = nrms[tid];
-    a.resnorms[v0 + tid] = nrm > 0.0 ? (float)(__builtin_sqrt(rn) / nrm) : 0.0f;
-  }
-  for (int i = tid; i < d; i += 256) {
-    double p[kIpV];
-#pragma unroll
-    for (int v = 0; v < kIpV; ++v) p[v] = 0.0;
-    for (int j = 0; j < d; ++j) {
-      const double s = (double)a.qjl_t[(size_t)j * d + i];
-#pragma unroll
-      for (int v = 0; v < kIpV; ++v) p[v] = fma(s, rs[v * kIpDMax + j], p[v]);
-    }
-#pragma unroll
-    for (int v = 0; v < kIpV; ++v) sb[v * kIpDMax + i] = p[v] >= 0.0 ? 1 : 0;
-  }
-  __syncthreads();
-  // Codes packed low bits first: bit t of a row is bit t % bits of code
-  // t / bits (a 3-bit code straddles two bytes where t crosses one).
-  for (int i = tid; i < nv * a.row_bytes; i += 256) {
-    const int v = i / a.row_bytes, b = i - v * a.row_bytes;
-    uint32_t byte = 0;
-    for (int e = 0; e < 8; ++e) {
-      const int t = 8 * b + e, j = t / a.bits;
-      if (j < d) byte |= (((uint32_t)cs[v * kIpDMax + j] >> (t - j * a.bits)) & 1u) << e;
-    }
-    a.codes[(size_t)(v0 + v) * a.row_bytes + b] = (uint8_t)byte;
-  }
-  for (int i = tid; i < nv * a.sign_bytes; i += 256) {
-    const int v = i / a.sign_bytes, b = i - v * a.sign_bytes;
-    uint32_t byte = 0;
-    for (int e = 0; e < 8; ++e) {
-      const int j = b * 8 + e;
-      if (j < d) byte |= (uint32_t)sb[v * kIpDMax + j] << e;
-    }
-    a.signs[(size_t)(v0 + v) * a.sign_bytes + b] = (uint8_t)byte;
-  }
-}
 
 // Query preparation of the inner-product layout: q' = R q and y = S q' (f64,
 // one fma chain per coordinate in k order), then eos_tq_ip_quant. These are

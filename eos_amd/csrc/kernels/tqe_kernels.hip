@@ -483,3 +483,277 @@ EOS_TQ_ENCODE_SPLIT(4)
 EOS_TQ_ENCODE_SPLIT(8)
 EOS_TQ_ENCODE_SPLIT(12)
 #undef EOS_TQ_ENCODE_SPLIT
+
+// ------------------------------------------------------- inner-product layout
+
+namespace {
+
+// The inner-product encode (the contract of eos_tq_ip_encode_device) with
+// both matrix products on v_mfma_f64_16x16x4_f64. That instruction adds its
+// four products to the accumulator one fma after another in K order, so a
+// chain of them over K is the contract's fma chain bit for bit (lane l of the
+// operands holds row or column l % 16 and K value l / 16; result element r
+// is row l / 16 + 4 r, column l % 16).
+// Workgroup: 16 NV vectors, all coordinates; wavefront w owns the 16-row tiles
+// w, w + 8, ... (at most TJ) of both products. Rotation: x in chunks of 64 K
+// values through two LDS stages, R^T fragments from global memory 16 K
+// values ahead. The residuals r = u - nrm c then stay in LDS as f64, the
+// second product's right operand, and one wavefront runs the ResNorm chains
+// over them beside its tiles. Rows of rs are 4 (mod 32) doubles apart: the 16
+// vectors x 4 K values of an operand read fall into different banks.
+// 200,000 x 384 at 3 bits: 10.96 -> 2.47 ms against f64 VALU chains (one workgroup
+// of 8 vectors per CU); bound by the f64 matrix rate (118
+// GFLOP; dependent chains of this instruction reach 62 TFLOP/s at two
+// wavefronts per SIMD).
+template <int NV, int TJ>
+struct EncodeIp {
+  static constexpr int BV = 16 * NV, KC = 64, XST = KC + 4, RST = 128 * TJ + 4;
+  static constexpr int kCodeRow = 64 * TJ;  // bytes: 8 TJ tiles x 16 codes of 4 bits
+  static constexpr int kSignRow = 16 * TJ;
+  static constexpr int kStage = 2 * BV * XST * 4;
+  static constexpr int kOut = BV * (kCodeRow + kSignRow);
+  struct Lds {
+    double rs[BV * RST];
+    double ncs[BV * 17];
+    double nrms[BV];
+    // x stages, then the packed codes and signs
+    uint32_t buf[(kStage > kOut ? kStage : kOut) / 4];
+  };
+
+  EOS_DEV static void run(const TqIpArgs& a, Lds& s) {
+    const int tid = threadIdx.x, lane = tid & 63, d = a.d, levels = 1 << a.bits;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 15, lk = lane >> 4;
+    const long long v0 = (long long)blockIdx.x * BV;
+    const int nv = (int)min((long long)BV, a.n - v0);
+    const int tiles = (d + 15) / 16;
+    float* const xs = reinterpret_cast<float*>(s.buf);
+
+    v4d acc[NV][TJ];
+    auto clear = [&]() {
+#pragma unroll
+      for (int n = 0; n < NV; ++n)
+#pragma unroll
+        for (int t = 0; t < TJ; ++t) acc[n][t] = v4d{0.0, 0.0, 0.0, 0.0};
+    };
+    // 16 K values (four steps) of the wavefront's rows of m [k][row].
+    auto load_m = [&](float (&f)[4][TJ], const float* m, int k0) {
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const int k = k0 + 4 * p + lk;
+        const float* row = m + (size_t)min(k, d - 1) * d;
+#pragma unroll
+        for (int t = 0; t < TJ; ++t) f[p][t] = row[min(16 * (wave + 8 * t) + lr, d - 1)];
+      }
+    };
+    auto steps = [&](const float (&f)[4][TJ], int k0, auto&& right) {
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const int k = k0 + 4 * p + lk;
+        double b[NV];
+#pragma unroll
+        for (int n = 0; n < NV; ++n) b[n] = right(n, k);
+#pragma unroll
+        for (int t = 0; t < TJ; ++t) {
+          const double r = (double)(k < d ? f[p][t] : 0.0f);
+#pragma unroll
+          for (int n = 0; n < NV; ++n)
+            acc[n][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(r, b[n], acc[n][t], 0, 0, 0);
+        }
+      }
+    };
+
+    // Staging thread t: values 4 (t % 16) .. + 3 of chunk c of vector t / 16.
+    const int sv = tid >> 4, sk = 4 * (tid & 15);
+    const bool stager = sv < BV;
+    float xr[4];
+    auto load_x = [&](int c) {
+      const float* src = a.x + (size_t)(v0 + min(sv, nv - 1)) * d;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) xr[e] = src[min(KC * c + sk + e, d - 1)];
+    };
+    auto store_x = [&](int c) {
+      if (!stager) return;
+      float4 v;
+      v.x = (sv < nv && KC * c + sk < d) ? xr[0] : 0.0f;
+      v.y = (sv < nv && KC * c + sk + 1 < d) ? xr[1] : 0.0f;
+      v.z = (sv < nv && KC * c + sk + 2 < d) ? xr[2] : 0.0f;
+      v.w = (sv < nv && KC * c + sk + 3 < d) ? xr[3] : 0.0f;
+      *reinterpret_cast<float4*>(&xs[((c & 1) * BV + sv) * XST + sk]) = v;
+    };
+    const int nchunk = (d + KC - 1) / KC;
+    load_x(0);
+    store_x(0);
+    load_x(1);
+    clear();
+    double ss = 0.0;
+    float fa[4][TJ], fb[4][TJ];
+    const bool rot = a.rot_t != nullptr;
+    if (rot) load_m(fa, a.rot_t, 0);
+    lds_barrier();
+    for (int c = 0; c < nchunk; ++c) {
+      const float* xc = xs + (c & 1) * BV * XST;
+      auto right = [&](int n, int k) { return (double)xc[(16 * n + lr) * XST + (k - KC * c)]; };
+      if (rot) {
+#pragma unroll
+        for (int h = 0; h < KC / 32; ++h) {
+          load_m(fb, a.rot_t, KC * c + 32 * h + 16);
+          steps(fa, KC * c + 32 * h, right);
+          load_m(fa, a.rot_t, KC * c + 32 * h + 32);
+          steps(fb, KC * c + 32 * h + 16, right);
+        }
+      }
+      // The norms' chains (vector = thread).
+      if (tid < BV) {
+#pragma unroll 4
+        for (int k = 0; k < KC; k += 4) {
+          const float4 v = *reinterpret_cast<const float4*>(&xc[tid * XST + k]);
+          ss = fma((double)v.x, (double)v.x, ss);
+          ss = fma((double)v.y, (double)v.y, ss);
+          ss = fma((double)v.z, (double)v.z, ss);
+          ss = fma((double)v.w, (double)v.w, ss);
+        }
+      }
+      store_x(c + 1);  // (past the last chunk: zeros nobody reads)
+      load_x(c + 2);
+      lds_barrier();
+    }
+    if (tid < BV) {
+      const double nrm = __builtin_sqrt(ss);
+      s.nrms[tid] = nrm;
+      if (tid < nv) a.norms[v0 + tid] = (float)nrm;
+      for (int l = 0; l < levels; ++l) s.ncs[tid * 17 + l] = nrm * ((double)a.cb_scale * (double)a.cb[l]);
+    }
+    if (!rot) {
+#pragma unroll
+      for (int n = 0; n < NV; ++n)
+#pragma unroll
+        for (int t = 0; t < TJ; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int v = 16 * n + lr, j = 16 * (wave + 8 * t) + lk + 4 * r;
+            acc[n][t][r] = v < nv && j < d ? (double)a.x[(size_t)(v0 + v) * d + j] : 0.0;
+          }
+    }
+    lds_barrier();
+
+    // Codes (the first level nearest u) and residuals.
+    uint8_t* const cbuf = reinterpret_cast<uint8_t*>(s.buf);
+    uint8_t* const sbuf = cbuf + BV * kCodeRow;
+#pragma unroll
+    for (int n = 0; n < NV; ++n) {
+      const double* nc = &s.ncs[(16 * n + lr) * 17];
+#pragma unroll
+      for (int t = 0; t < TJ; ++t) {
+        if (wave + 8 * t >= tiles) continue;
+        double bd[4];
+        int best[4];
+        const double n0 = nc[0];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          bd[r] = fabs(acc[n][t][r] - n0);
+          best[r] = 0;
+        }
+        for (int l = 1; l < levels; ++l) {
+          const double nl = nc[l];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const double dv = fabs(acc[n][t][r] - nl);
+            if (dv < bd[r]) {
+              bd[r] = dv;
+              best[r] = l;
+            }
+          }
+        }
+        uint64_t pk = 0;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int j = 16 * (wave + 8 * t) + lk + 4 * r;
+          const double res = acc[n][t][r] - nc[best[r]];
+          s.rs[(16 * n + lr) * RST + j] = j < d ? res : 0.0;
+          if (j < d) pk |= (uint64_t)best[r] << (a.bits * (lk + 4 * r));
+        }
+        // The tile's 16 codes are 2 bits-many bytes: group lk writes two.
+        uint32_t lo = (uint32_t)pk, hi = (uint32_t)(pk >> 32);
+        lo |= (uint32_t)__shfl_xor((int)lo, 16);
+        hi |= (uint32_t)__shfl_xor((int)hi, 16);
+        lo |= (uint32_t)__shfl_xor((int)lo, 32);
+        hi |= (uint32_t)__shfl_xor((int)hi, 32);
+        if (lk < a.bits)
+          *reinterpret_cast<uint16_t*>(&cbuf[(16 * n + lr) * kCodeRow + (wave + 8 * t) * 2 * a.bits + 2 * lk]) =
+              (uint16_t)((lk & 2 ? hi : lo) >> (lk & 1 ? 16 : 0));
+      }
+    }
+    lds_barrier();
+
+    if (wave == 7 && lane < nv) {
+      double rn = 0.0;
+      const double* r = &s.rs[lane * RST];
+#pragma unroll 8
+      for (int j = 0; j < d; ++j) rn = fma(r[j], r[j], rn);
+      const double nrm = s.nrms[lane];
+      a.resnorms[v0 + lane] = nrm > 0.0 ? (float)(__builtin_sqrt(rn) / nrm) : 0.0f;
+    }
+    clear();
+    auto right = [&](int n, int k) { return k < d ? s.rs[(16 * n + lr) * RST + k] : 0.0; };
+    load_m(fa, a.qjl_t, 0);
+    for (int k0 = 0; k0 < d; k0 += 32) {
+      load_m(fb, a.qjl_t, k0 + 16);
+      steps(fa, k0, right);
+      load_m(fa, a.qjl_t, k0 + 32);
+      if (k0 + 16 < d) steps(fb, k0 + 16, right);
+    }
+#pragma unroll
+    for (int n = 0; n < NV; ++n)
+#pragma unroll
+      for (int t = 0; t < TJ; ++t) {
+        if (wave + 8 * t >= tiles) continue;
+        uint32_t m = 0;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = 16 * (wave + 8 * t) + lk + 4 * r;
+          m |= (i < d && acc[n][t][r] >= 0.0 ? 1u : 0u) << (lk + 4 * r);
+        }
+        m |= (uint32_t)__shfl_xor((int)m, 16);
+        m |= (uint32_t)__shfl_xor((int)m, 32);
+        if (lk == 0)
+          *reinterpret_cast<uint16_t*>(&sbuf[(16 * n + lr) * kSignRow + (wave + 8 * t) * 2]) = (uint16_t)m;
+      }
+    lds_barrier();
+    auto put = [&](uint8_t* dst, int bytes, const uint8_t* src, int pitch) {
+      if ((bytes & 3) == 0 && (reinterpret_cast<uintptr_t>(dst) & 3) == 0) {
+        const int nw = bytes >> 2;
+        for (int i = tid; i < nv * nw; i += 512) {
+          const int v = i / nw, b = i - v * nw;
+          reinterpret_cast<uint32_t*>(dst + (size_t)v * bytes)[b] =
+              *reinterpret_cast<const uint32_t*>(src + v * pitch + 4 * b);
+        }
+      } else {
+        for (int i = tid; i < nv * bytes; i += 512) {
+          const int v = i / bytes, b = i - v * bytes;
+          dst[(size_t)v * bytes + b] = src[v * pitch + b];
+        }
+      }
+    };
+    put(a.codes + (size_t)v0 * a.row_bytes, a.row_bytes, cbuf, kCodeRow);
+    put(a.signs + (size_t)v0 * a.sign_bytes, a.sign_bytes, sbuf, kSignRow);
+  }
+};
+
+}  // namespace
+
+// 16 NV vectors per workgroup, up to 128 TJ coordinates.
+#define EOS_TQ_ENCODE_IP(NV, TJ)                                                        \
+  extern "C" __global__ __launch_bounds__(512) void eos_tq_encode_ip_t##TJ(TqIpArgs a) { \
+    __shared__ __attribute__((aligned(16))) EncodeIp<NV, TJ>::Lds lds;                  \
+    EncodeIp<NV, TJ>::run(a, lds);                                                      \
+  }
+EOS_TQ_ENCODE_IP(2, 1)
+EOS_TQ_ENCODE_IP(2, 2)
+EOS_TQ_ENCODE_IP(2, 3)
+EOS_TQ_ENCODE_IP(2, 4)
+EOS_TQ_ENCODE_IP(1, 5)
+EOS_TQ_ENCODE_IP(1, 6)
+EOS_TQ_ENCODE_IP(1, 7)
+EOS_TQ_ENCODE_IP(1, 8)
+#undef EOS_TQ_ENCODE_IP
