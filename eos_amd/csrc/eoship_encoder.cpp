@@ -3,7 +3,9 @@
 // 101-197) on the runtime stream:
 //   eos_enc_pack        active positions -> contiguous rows per sequence
 //   eos_enc_embed       token + position + type, affine LayerNorm
-//   per layer:  eos_enc_gemm_t* (QKV) -> eos_enc_attn_hd* -> eos_enc_gemm_t*
+//   per layer (small batches: eos_enc_lin8_* QKV -> attention -> eos_enc_lin16 O
+//   -> eos_enc_lin8_* FFN up -> eos_enc_lin16 FFN down, LayerNorms inside):
+//               eos_enc_gemm_t* (QKV) -> eos_enc_attn_hd* -> eos_enc_gemm_t*
 //               (O + residual) -> eos_enc_ln -> eos_enc_gemm_t* (FFN up + GELU)
 //               -> eos_enc_gemm_t* (FFN down + residual) -> eos_enc_ln
 //   eos_enc_pool        masked mean pool + L2 normalize
@@ -58,6 +60,7 @@ struct DevLayer {
   uint16_t* w_of = nullptr;
   int8_t* w_1f = nullptr;
   uint16_t* w_2f = nullptr;
+  int8_t* w_qkvf = nullptr;  // the QKV codes likewise (small batches)
   // General-shape path: int8 codes of the O and FFN-down weights.
   int8_t* w_o8 = nullptr;
   int8_t* w_28 = nullptr;
@@ -99,6 +102,7 @@ struct EosHipEncoder {
   size_t cap_rows = 0;
   int cap_batch = 0;
   uint16_t *h = nullptr, *qkv = nullptr, *ctx = nullptr, *mid = nullptr;
+  uint16_t* hb = nullptr;  // small batches: the layer input rows
   // int8 copy of h with one scale per row (BERT family: QKV and FFN-up run on
   // int8 MFMA with these as activations)
   int8_t* h8 = nullptr;
@@ -122,7 +126,7 @@ struct EosHipEncoder {
   ~EosHipEncoder() {
     for (void* p : owned)
       if (p) hipFree(p);
-    void* act[] = {h,     qkv,     ctx,     mid,   h8,    hs,   pool_part, vt, row_b,
+    void* act[] = {h,     qkv,     ctx,     mid,   hb,    h8,    hs,   pool_part, vt, row_b,
                    row_t, seq_off, seq_cnt, seq_q, total, status, io,   hf,        h1f, qkvf,
                    ctxf,  midf,    seq_order};
     for (void* p : act)
@@ -198,17 +202,35 @@ struct EosHipEncoder {
   // to batch * (tokens + 7) rows.
   static size_t row_capacity(int batch, int tokens) { return (size_t)batch * (tokens + 7); }
 
+  // BERT family: batches of up to this many packed rows run their linear
+  // layers as eos_enc_lin8 / lin16 launches, larger ones as the wide GEMM and
+  // the tail (128, 256: the unfused GEMMs). The tail takes as long for one row
+  // block as for one on every CU; the small launches grow with the rows. Where
+  // the two meet, 4 layers, us per forward (small against large path):
+  //   H 128: 32,768 rows 385 / 410     H 256: 8,192 283 / 308, 16,384 421 / 415
+  //   H 384: 4,096 296 / 356, 8,192 448 / 395   H 512: 4,096 371 / 411, 8,192 613 / 460
+  //   H 768: 4,096 650 / 725, 8,192 1091 / 830  (24 rows: H 384 165 / 310, H 768 241 / 679)
+  int lin_rows() const {
+    switch (desc.hidden) {
+      case 128: return 40960;
+      case 256: return 12288;
+      case 384: return 5632;
+      case 512: return 5120;
+      default: return 4864;
+    }
+  }
+
   int ensure_activations(int batch, int tokens, char** err) {
     const size_t rows = row_capacity(batch, tokens);
     if (rows <= cap_rows && batch <= cap_batch) return 0;
-    void* act[] = {h,     qkv,   ctx,     mid,     h8,    hs,     pool_part, vt,  row_b, row_t,
+    void* act[] = {h,     qkv,   ctx,     mid,     hb,    h8,    hs,     pool_part, vt,  row_b, row_t,
                    seq_off, seq_cnt, seq_q, total, status, hf,  h1f,       qkvf, ctxf, midf,
                    seq_order};
     for (void* p : act)
       if (p) hipFree(p);
     hf = h1f = qkvf = ctxf = midf = nullptr;
     seq_order = nullptr;
-    h = qkv = ctx = mid = nullptr;
+    h = qkv = ctx = mid = hb = nullptr;
     h8 = nullptr;
     hs = nullptr;
     pool_part = nullptr;
@@ -221,6 +243,8 @@ struct EosHipEncoder {
         rt->alloc(rows * 3 * H * 2, reinterpret_cast<void**>(&qkv), err) ||
         rt->alloc(rows * H * 2, reinterpret_cast<void**>(&ctx), err) ||
         rt->alloc(rows * F * 2, reinterpret_cast<void**>(&mid), err) ||
+        (family == 0 && !general &&
+         rt->alloc(std::min(rows, (size_t)lin_rows()) * H * 2, reinterpret_cast<void**>(&hb), err)) ||
         rt->alloc(rows * H, reinterpret_cast<void**>(&h8), err) ||
         rt->alloc(rows * 4, reinterpret_cast<void**>(&hs), err) ||
         // chunks of any later shape within the caps: batch' * ceil(tokens' /
@@ -432,9 +456,44 @@ struct EosHipEncoder {
       snprintf(tail_buf, sizeof(tail_buf), "eos_enc_tail_r%d_h%d_g%d", tail_bm / 32, H, desc.gelu);
       tail_name = tail_buf;
     }
+    const bool small = a8 && fused_tail && max_rows <= lin_rows();
+    auto lin = [&](const char* kind, EncLinArgs l, const char* label) {
+      l.rows = total;
+      l.max_rows = max_rows;
+      l.eps = desc.ln_eps;
+      char name[40];
+      const bool l8 = kind[0] == '8';
+      snprintf(name, sizeof(name), l8 ? "eos_enc_lin8_h%d_g%s" : "eos_enc_lin16", H, kind + 1);
+      const int bm = l8 ? 32 : 64, bn = l8 ? 256 : 128;
+      const unsigned grid = (unsigned)((max_rows + bm - 1) / bm) * (unsigned)((l.n + bn - 1) / bn);
+      return rt->launch(name, dim3(grid), dim3(l8 ? 512 : 256), 0, &l, err, label);
+    };
+    const DevLayer* prev = nullptr;
     for (const DevLayer& L : layers) {
       // Q and K rows into qkv, V feature-major into vt.
-      if (gemm(h, L.w_qkv, a8 ? L.w_qkv8 : nullptr, L.s_qkv, L.b_qkv, qkv, nullptr, 3 * H, H, 0,
+      if (small) {
+        // The first layer's rows come quantized from the embedding; later
+        // ones are the last layer's sums, normalized here (rows to hb).
+        EncLinArgs q{};
+        if (prev == nullptr) {
+          q.x8 = h8;
+          q.xs = hs;
+        } else {
+          q.x = h;
+          q.gamma = prev->g2;
+          q.beta = prev->be2;
+          q.ln_out = hb;
+        }
+        q.w = L.w_qkvf;
+        q.s = L.s_qkv;
+        q.b = L.b_qkv;
+        q.out = qkv;
+        q.n = 3 * H;
+        q.vt = vt;
+        q.vt_col0 = 2 * H;
+        q.vt_ld = vt_ld;
+        if (lin("80", q, "enc_gemm_qkv") != 0) return 1;
+      } else if (gemm(h, L.w_qkv, a8 ? L.w_qkv8 : nullptr, L.s_qkv, L.b_qkv, qkv, nullptr, 3 * H, H, 0,
                "enc_gemm_qkv", vt) != 0)
         return 1;
       const double log2e = 1.4426950408889634;
@@ -450,6 +509,41 @@ struct EosHipEncoder {
                      dim3((tokens + qpw - 1) / qpw, nh, batch), dim3(wide ? 768 : 256), 0, &at,
                      err) != 0)
         return 1;
+      if (small) {
+        EncLinArgs o{};
+        o.x = ctx;
+        o.w = L.w_of;
+        o.s = L.s_o;
+        o.b = L.b_o;
+        o.res = prev == nullptr ? h : hb;
+        o.out = h;
+        o.n = o.k = H;
+        EncLinArgs u{};
+        u.x = h;
+        u.gamma = L.g1;
+        u.beta = L.be1;
+        u.ln_out = ctx;
+        u.w = L.w_1f;
+        u.s = L.s_1;
+        u.b = L.b_1;
+        u.out = mid;
+        u.n = F;
+        EncLinArgs dn{};
+        dn.x = mid;
+        dn.w = L.w_2f;
+        dn.s = L.s_2;
+        dn.b = L.b_2;
+        dn.res = ctx;
+        dn.out = h;
+        dn.n = H;
+        dn.k = F;
+        if (lin("16", o, "enc_gemm_o") != 0 ||
+            lin(desc.gelu == 1 ? "81" : "82", u, "enc_gemm_ffn_up") != 0 ||
+            lin("16", dn, "enc_gemm_ffn_down") != 0)
+          return 1;
+        prev = &L;
+        continue;
+      }
       if (tail_name != nullptr) {
         EncTailArgs tl{ctx,    h,      mid,    h8,     hs,     L.w_of, L.s_o,    L.b_o,     L.g1,
                        L.be1,  L.w_1f, L.s_1,  L.b_1,  L.w_2f, L.s_2,    L.b_2,     L.g2,
@@ -490,6 +584,12 @@ struct EosHipEncoder {
                "enc_gemm_ffn_up") != 0 ||
           gemm(mid, L.w_2, nullptr, L.s_2, L.b_2, h, h, H, F, 3, "enc_gemm_ffn_down") != 0 ||
           layer_norm(L.g2, L.be2) != 0)
+        return 1;
+    }
+    if (prev != nullptr) {
+      EncLnArgs l{h, prev->g2, prev->be2, total, max_rows, H, desc.ln_eps, nullptr, nullptr};
+      if (rt->launch("eos_enc_ln", dim3((unsigned)((max_rows + 3) / 4)), dim3(256), 0, &l, err,
+                     "enc_ln") != 0)
         return 1;
     }
     const int nchunk = (tokens + kPoolChunk - 1) / kPoolChunk;
@@ -593,8 +693,9 @@ int eoship_encoder_bind(EosHipRuntime* rt, const EosHipEncoderDesc* desc, const 
     if (general && (enc->upload(&d.w_o8, s.w_o, (size_t)H * H, err) ||
                     enc->upload(&d.w_28, s.w_2, (size_t)H * F, err)))
       return fail();
-    if ((H == 384 || H == 512 || H == 768) &&
-        (enc->upload_frag16(&d.w_of, s.w_o, H, H, err) ||
+    if (!general &&
+        (enc->upload_frag8(&d.w_qkvf, s.w_qkv, 3 * H, H, err) ||
+         enc->upload_frag16(&d.w_of, s.w_o, H, H, err) ||
          enc->upload_frag8(&d.w_1f, s.w_1, F, H, err) ||
          enc->upload_frag16(&d.w_2f, s.w_2, H, F, err)))
       return fail();

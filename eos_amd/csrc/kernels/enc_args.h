@@ -123,6 +123,30 @@ struct EncTailArgs {
   int row0, row_cap;
 };
 
+// Small-batch linear layers (eos_enc_lin8_*, eos_enc_lin16), weights in the
+// tail's fragment order. lin8: x [rows][hidden] f16 rows that the kernel
+// normalizes first (gamma, beta, eps; the f16 rows also go to ln_out), or,
+// with x NULL, rows x8 / xs already quantized; int8 x int8 products; out
+// [rows][n] f16, for QKV the columns from vt_col0 on to vt[col - vt_col0][row].
+// lin16: x [rows][k] f16, out = x W^T s + b + res.
+struct EncLinArgs {
+  const uint16_t* x;
+  const int8_t* x8;        // [rows][hidden]
+  const float* xs;         // [rows]
+  const float* gamma;
+  const float* beta;
+  uint16_t* ln_out;        // [rows][hidden]
+  const void* w;           // fragment order
+  const float* s;          // [n]
+  const float* b;          // [n]
+  const uint16_t* res;     // lin16: [rows][n]
+  uint16_t* out;
+  uint16_t* vt;
+  const int32_t* rows;     // device row count
+  int max_rows, n, k, vt_col0, vt_ld;
+  float eps;
+};
+
 // In-place affine LayerNorm of h [rows][hidden] f16 (hidden % 8 == 0, <= 1024).
 struct EncLnArgs {
   uint16_t* h;

@@ -1477,6 +1477,232 @@ EOS_TAIL_KERNEL(1, 768, 1)
 EOS_TAIL_KERNEL(1, 768, 2)
 #undef EOS_TAIL_KERNEL
 
+// ------------------------------------------------- small-batch linear layers
+
+namespace {
+
+// The BERT layer for batches whose row blocks cannot fill the chip as fused
+// tails (a 96-row tail block runs a whole layer's weights on one CU: 24 rows
+// at H 384, 61 us per layer on one block): every linear layer spread over row
+// tiles x column blocks, the LayerNorms in the prologue of the layer that
+// reads them. The sums run in the same K order on the same instructions, and
+// every value is rounded where the tail and the wide GEMMs round it, so the
+// embeddings do not depend on which path a batch takes.
+//
+// Workgroup: 32 rows x 256 columns, wavefront w the columns [32 w, + 32) of
+// the block. All of a wavefront's weights (H / 32 KB) are requested before the
+// LayerNorm, which 8 wavefronts run on 4 rows each. Every column block of a
+// row tile repeats the LayerNorm; the first writes its rows out.
+// EPI 0: QKV, 1: erf GELU, 2: tanh GELU.
+template <int H, int EPI>
+struct Lin8 {
+  static constexpr int BM = 32, QS = H + 16, KS = H / 32;
+  struct Lds {
+    int8_t q8[BM * QS];
+    float rsc[BM];
+    uint16_t dump[8][H];  // LayerNorm rows another column block writes out
+  };
+  EOS_DEV static void run(const EncLinArgs& a, Lds& s) {
+    const int ncb = (a.n + 255) / 256;
+    const int m0 = (int)(blockIdx.x / ncb) * BM, cb = blockIdx.x % ncb;
+    const int rows = *a.rows;
+    if (m0 >= rows) return;
+    const int lane = threadIdx.x & 63, g = lane >> 5, l32 = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n0 = 256 * cb + 32 * wave;
+    const bool active = n0 < a.n;
+    const v4i* wsrc = reinterpret_cast<const v4i*>(a.w) +
+                      (size_t)(active ? n0 / 32 : 0) * KS * 64 + lane;
+    v4i wf[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) wf[ks] = wsrc[64 * ks];
+    if (a.x != nullptr) {
+      LnParams<H> p;
+      ln_params<H>(a.gamma, a.beta, lane, p);
+      const uint16_t* yin[4];
+      uint16_t* yout[4];
+      int8_t* q8[4];
+      float* qs[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int m = 4 * wave + r;
+        yin[r] = a.x + (size_t)min(m0 + m, a.max_rows - 1) * H;
+        yout[r] = cb == 0 && m0 + m < rows ? a.ln_out + (size_t)(m0 + m) * H : s.dump[wave];
+        q8[r] = &s.q8[m * QS];
+        qs[r] = &s.rsc[m];
+      }
+      ln_rows<H, 4>(yin, p, a.eps, lane, yout, q8, qs);
+    } else {
+      constexpr int PER = BM * H / 16;  // 16-byte pieces
+      for (int i = threadIdx.x; i < PER; i += 512) {
+        const int r = i / (H / 16), c = i % (H / 16);
+        *reinterpret_cast<v4i*>(&s.q8[r * QS + 16 * c]) = *reinterpret_cast<const v4i*>(
+            a.x8 + (size_t)min(m0 + r, a.max_rows - 1) * H + 16 * c);
+      }
+      if (threadIdx.x < BM) s.rsc[threadIdx.x] = a.xs[min(m0 + (int)threadIdx.x, a.max_rows - 1)];
+    }
+    __syncthreads();
+    if (!active) return;
+    const bool tr = EPI == 0 && a.vt != nullptr && n0 >= a.vt_col0;
+    v16i acc = v16i{0};
+    auto frag = [&](int ks) {
+      return *reinterpret_cast<const v4i*>(&s.q8[l32 * QS + 32 * ks + 16 * g]);
+    };
+    if (tr) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(frag(ks), wf[ks], acc, 0, 0, 0);
+      // A lane's results lie along a column: 4 rows per 8-byte store.
+      const float sc = a.s[n0 + l32], bi = a.b[n0 + l32];
+      uint16_t* col = a.vt + (size_t)(n0 + l32 - a.vt_col0) * a.vt_ld + m0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int r = 8 * q + 4 * g;
+        if (m0 + r >= rows) continue;  // rows is a multiple of 8
+        v4h o;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          o[t] = (_Float16)__builtin_fmaf((float)acc[4 * q + t], sc * s.rsc[r + t], bi);
+        *reinterpret_cast<v4h*>(col + r) = o;
+      }
+      return;
+    }
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(wf[ks], frag(ks), acc, 0, 0, 0);
+    if (m0 + l32 >= rows) return;
+    const float rs = s.rsc[l32];
+    uint16_t* orow = a.out + (size_t)(m0 + l32) * a.n;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int n = n0 + 8 * q + 4 * g;
+      const float4 sc = *reinterpret_cast<const float4*>(a.s + n);
+      const float4 bi = *reinterpret_cast<const float4*>(a.b + n);
+      float v[4] = {__builtin_fmaf((float)acc[4 * q], sc.x * rs, bi.x),
+                    __builtin_fmaf((float)acc[4 * q + 1], sc.y * rs, bi.y),
+                    __builtin_fmaf((float)acc[4 * q + 2], sc.z * rs, bi.z),
+                    __builtin_fmaf((float)acc[4 * q + 3], sc.w * rs, bi.w)};
+      v4h o;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        o[t] = (_Float16)(EPI == 1 ? gelu_erf_fast(v[t]) : EPI == 2 ? gelu(v[t], 2) : v[t]);
+      *reinterpret_cast<v4h*>(orow + n) = o;
+    }
+  }
+};
+
+// The O and FFN-down projections of small batches: 64 rows x 128 columns per
+// workgroup, wavefront w the columns [32 w, + 32), K in chunks of 128 through
+// two LDS stages (one barrier per chunk), weights eight K steps ahead.
+// out = acc s + b + res, rounded once (out may alias res).
+constexpr int kLinK = 128;
+struct Lin16Lds {
+  uint16_t a[2][64 * (kLinK + 8)];
+};
+EOS_DEV void lin16_body(const EncLinArgs& a, Lin16Lds& s) {
+  constexpr int BM = 64, RT = 2, AS = kLinK + 8, PER = BM * kLinK / 8 / 256;
+  const int ncb = a.n / 128;
+  const int m0 = (int)(blockIdx.x / ncb) * BM, n0 = (blockIdx.x % ncb) * 128;
+  const int rows = *a.rows;
+  if (m0 >= rows) return;
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, l32 = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nw = n0 + 32 * wave, nk = a.k / kLinK;
+  const v8h* wsrc = reinterpret_cast<const v8h*>(a.w) + (size_t)(nw / 32) * (a.k / 16) * 64 + lane;
+  v8h wq[8];
+#pragma unroll
+  for (int p = 0; p < 8; ++p) wq[p] = wsrc[64 * p];
+  v4i st[PER];
+  auto load = [&](int c) {
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int i = tid + 256 * u, r = i / (kLinK / 8), k8 = i % (kLinK / 8);
+      st[u] = *reinterpret_cast<const v4i*>(a.x + (size_t)min(m0 + r, a.max_rows - 1) * a.k +
+                                            kLinK * c + 8 * k8);
+    }
+  };
+  auto store = [&](int b) {
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int i = tid + 256 * u, r = i / (kLinK / 8), k8 = i % (kLinK / 8);
+      *reinterpret_cast<v4i*>(&s.a[b][r * AS + 8 * k8]) = st[u];
+    }
+  };
+  load(0);
+  // The residual is requested with the first chunk.
+  v4h res[RT][4];
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      res[i][q] = *reinterpret_cast<const v4h*>(
+          a.res + (size_t)min(m0 + 32 * i + l32, a.max_rows - 1) * a.n + nw + 8 * q + 4 * g);
+  store(0);
+  load(min(1, nk - 1));
+  __syncthreads();
+  v16f acc[RT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i) acc[i] = v16f{0};
+  for (int c = 0; c < nk; ++c) {
+    const uint16_t* A = s.a[c & 1];
+    const int nx = min(c + 1, nk - 1) * 8;  // the next chunk's first K step
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) {
+      v8h bf[RT];
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+        bf[i] = *reinterpret_cast<const v8h*>(&A[(32 * i + l32) * AS + 16 * kk + 8 * g]);
+      const v8h af = wq[kk];
+      wq[kk] = wsrc[64 * (size_t)(nx + kk)];
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, bf[i], acc[i], 0, 0, 0);
+    }
+    store((c + 1) & 1);
+    load(min(c + 2, nk - 1));
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < RT; ++i) {
+    const int row = m0 + 32 * i + l32;
+    if (row >= rows) continue;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int n = nw + 8 * q + 4 * g;
+      const float4 sc = *reinterpret_cast<const float4*>(a.s + n);
+      const float4 bi = *reinterpret_cast<const float4*>(a.b + n);
+      float v[4] = {__builtin_fmaf(acc[i][4 * q], sc.x, bi.x),
+                    __builtin_fmaf(acc[i][4 * q + 1], sc.y, bi.y),
+                    __builtin_fmaf(acc[i][4 * q + 2], sc.z, bi.z),
+                    __builtin_fmaf(acc[i][4 * q + 3], sc.w, bi.w)};
+      v4h o;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) o[t] = (_Float16)(v[t] + (float)res[i][q][t]);
+      *reinterpret_cast<v4h*>(a.out + (size_t)row * a.n + n) = o;
+    }
+  }
+}
+
+}  // namespace
+
+#define EOS_LIN8_KERNEL(H, G)                                                              \
+  extern "C" __global__ __launch_bounds__(512) void eos_enc_lin8_h##H##_g##G(EncLinArgs a) { \
+    __shared__ __attribute__((aligned(16))) Lin8<H, G>::Lds lds;                           \
+    Lin8<H, G>::run(a, lds);                                                               \
+  }
+#define EOS_LIN8_KERNELS(H) EOS_LIN8_KERNEL(H, 0) EOS_LIN8_KERNEL(H, 1) EOS_LIN8_KERNEL(H, 2)
+EOS_LIN8_KERNELS(128)
+EOS_LIN8_KERNELS(256)
+EOS_LIN8_KERNELS(384)
+EOS_LIN8_KERNELS(512)
+EOS_LIN8_KERNELS(768)
+#undef EOS_LIN8_KERNELS
+#undef EOS_LIN8_KERNEL
+extern "C" __global__ __launch_bounds__(256) void eos_enc_lin16(EncLinArgs a) {
+  __shared__ __attribute__((aligned(16))) Lin16Lds lds;
+  lin16_body(a, lds);
+}
+
 // --------------------------------------------------------------- attention
 
 // Flash-style attention in transposed form: each wavefront owns 32 queries of
