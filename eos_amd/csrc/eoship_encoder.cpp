@@ -75,9 +75,8 @@ struct EosHipEncoder {
   // family (token + role with RoPE, normalize per row then pool, optional
   // output projection `proj` [hidden][odim] f32).
   int family = 0;
-  // BERT family at hidden 384 / 512 / 768: O projection through the second
-  // LayerNorm as one kernel per row block (eos_enc_tail_*); otherwise, or
-  // when switched off, the unfused GEMM + LayerNorm launches.
+  // BERT family: the fused layer paths (tail kernels, small-batch linear
+  // layers); when switched off, GEMM + LayerNorm launches throughout.
   bool fused_tail = true;
   // BERT family at a hidden width or head dim the MFMA kernels do not take
   // (e.g. hidden 16, head dim 4): the f32 eos_enc_gen_* kernels run every
@@ -202,23 +201,22 @@ struct EosHipEncoder {
   // to batch * (tokens + 7) rows.
   static size_t row_capacity(int batch, int tokens) { return (size_t)batch * (tokens + 7); }
 
-  // BERT family: batches of up to this many packed rows run their linear
-  // layers as eos_enc_lin8 / lin16 launches, larger ones as the wide GEMM and
-  // the tail (128, 256: the unfused GEMMs). The tail takes as long for one row
-  // block as for one on every CU; the small launches grow with the rows. Where
-  // the two meet, 4 layers, us per forward (small against large path):
-  //   H 128: 32,768 rows 385 / 410     H 256: 8,192 283 / 308, 16,384 421 / 415
-  //   H 384: 4,096 296 / 356, 8,192 448 / 395   H 512: 4,096 371 / 411, 8,192 613 / 460
-  //   H 768: 4,096 650 / 725, 8,192 1091 / 830  (24 rows: H 384 165 / 310, H 768 241 / 679)
-  int lin_rows() const {
-    switch (desc.hidden) {
-      case 128: return 40960;
-      case 256: return 12288;
-      case 384: return 5632;
-      case 512: return 5120;
-      default: return 4864;
-    }
-  }
+  // Which launches run a BERT layer of a batch of up to `rows` packed rows
+  // (4 layers, us per forward; all give the same bits):
+  //  - eos_enc_lin8 / lin16, LayerNorms inside, up to lin_rows(): rows H^2 <=
+  //    5.5e8. Their column blocks repeat the LayerNorm and re-read the rows,
+  //    which the wide GEMM after a LayerNorm launch does not: H 384 2,048
+  //    rows 226 against 258, 4,096 307 / 289; H 768 1,024 311 / 301, 2,048
+  //    424 / 359; H 256 8,192 283 / 300; H 128 32,768 385 / 404.
+  //  - the fused tail (H 384, 512) above kTailRows. One row block takes it as
+  //    long as one on every CU: H 384 4,096 rows 289 against 356, 8,192 390 /
+  //    396, 32,768 1042 / 860; H 512 4,096 353 / 411, 8,192 473 / 460. At H 768
+  //    a 32-row block carries all 8 MB of weights and the GEMMs win at every
+  //    size (8,192 rows 792 against 833, 32,768 2499 / 3133).
+  //  - LayerNorm, GEMM launches otherwise (and lin16 for O and FFN down while
+  //    their tiles are few, below).
+  static constexpr int kTailRows = 7680;
+  size_t lin_rows() const { return (size_t)550000000 / ((size_t)desc.hidden * desc.hidden); }
 
   int ensure_activations(int batch, int tokens, char** err) {
     const size_t rows = row_capacity(batch, tokens);
@@ -244,7 +242,7 @@ struct EosHipEncoder {
         rt->alloc(rows * H * 2, reinterpret_cast<void**>(&ctx), err) ||
         rt->alloc(rows * F * 2, reinterpret_cast<void**>(&mid), err) ||
         (family == 0 && !general &&
-         rt->alloc(std::min(rows, (size_t)lin_rows()) * H * 2, reinterpret_cast<void**>(&hb), err)) ||
+         rt->alloc(std::min(rows, lin_rows()) * H * 2, reinterpret_cast<void**>(&hb), err)) ||
         rt->alloc(rows * H, reinterpret_cast<void**>(&h8), err) ||
         rt->alloc(rows * 4, reinterpret_cast<void**>(&hs), err) ||
         // chunks of any later shape within the caps: batch' * ceil(tokens' /
@@ -447,28 +445,56 @@ struct EosHipEncoder {
       return rt->launch("eos_enc_ln", dim3((unsigned)((max_rows + 3) / 4)), dim3(256), 0, &l, err,
                         "enc_ln");
     };
+    const bool wide_tail = a8 && fused_tail && (H == 384 || H == 512) && F <= 4 * H &&
+                           max_rows > kTailRows;
+    const bool small = a8 && fused_tail && !wide_tail && (size_t)max_rows <= lin_rows();
     // Fused tail: the largest row block whose LDS fits the hidden width.
     const char* tail_name = nullptr;
     char tail_buf[48];
     int tail_bm = 0;
-    if (a8 && fused_tail && (H == 384 || H == 512 || H == 768) && F <= 4 * H) {
-      tail_bm = H == 384 ? 96 : H == 512 ? 64 : 32;
+    if (wide_tail) {
+      tail_bm = H == 384 ? 96 : 64;
       snprintf(tail_buf, sizeof(tail_buf), "eos_enc_tail_r%d_h%d_g%d", tail_bm / 32, H, desc.gelu);
       tail_name = tail_buf;
     }
-    const bool small = a8 && fused_tail && max_rows <= lin_rows();
-    auto lin = [&](const char* kind, EncLinArgs l, const char* label) {
+    auto lin8 = [&](EncLinArgs l, int epi, const char* label) {
       l.rows = total;
       l.max_rows = max_rows;
       l.eps = desc.ln_eps;
-      char name[40];
-      const bool l8 = kind[0] == '8';
-      snprintf(name, sizeof(name), l8 ? "eos_enc_lin8_h%d_g%s" : "eos_enc_lin16", H, kind + 1);
-      const int bm = l8 ? 32 : 64, bn = l8 ? 256 : 128;
-      const unsigned grid = (unsigned)((max_rows + bm - 1) / bm) * (unsigned)((l.n + bn - 1) / bn);
-      return rt->launch(name, dim3(grid), dim3(l8 ? 512 : 256), 0, &l, err, label);
+      char name[32];
+      snprintf(name, sizeof(name), "eos_enc_lin8_h%d_g%d", H, epi);
+      return rt->launch(name, dim3((unsigned)((max_rows + 31) / 32 * ((l.n + 255) / 256))), dim3(512),
+                        0, &l, err, label);
     };
-    const DevLayer* prev = nullptr;
+    // O and FFN down (x W^T s + b + res). 64-row x 128-column tiles of lin16
+    // up to 5/4 per CU, 32-row ones while those would leave half the CUs
+    // idle, the 128 x 128 GEMM beyond (FFN down, H 768: 1,024 rows 17.9 / 22.9
+    // / 27 us with 32-row tiles, 64-row tiles, the GEMM; 2,048 rows 26.2 / 24.6 /
+    // 32.5; 4,096 rows 43.6 / 38.2 / 32.6). The row count is the batch's
+    // capacity; padding leaves fewer.
+    auto project = [&](const uint16_t* x, const uint16_t* wf, const uint16_t* w, const float* sc,
+                       const float* b, const uint16_t* res, int k, const char* label) {
+      const int tiles = (max_rows + 63) / 64 * (H / 128);
+      if (wf == nullptr || !fused_tail || (!small && 4 * tiles > 5 * rt->compute_units))
+        return gemm(x, w, nullptr, sc, b, h, res, H, k, 3, label);
+      EncLinArgs l{};
+      l.x = x;
+      l.w = wf;
+      l.s = sc;
+      l.b = b;
+      l.res = res;
+      l.out = h;
+      l.rows = total;
+      l.max_rows = max_rows;
+      l.n = H;
+      l.k = k;
+      const bool r1 = 2 * tiles <= rt->compute_units;
+      const int bm = r1 ? 32 : 64;
+      return rt->launch(r1 ? "eos_enc_lin16_r1" : "eos_enc_lin16_r2",
+                        dim3((unsigned)((max_rows + bm - 1) / bm * (H / 128))), dim3(256), 0, &l, err,
+                        label);
+    };
+    const DevLayer* prev = nullptr;  // small: the layer whose second LayerNorm is still to come
     for (const DevLayer& L : layers) {
       // Q and K rows into qkv, V feature-major into vt.
       if (small) {
@@ -492,10 +518,11 @@ struct EosHipEncoder {
         q.vt = vt;
         q.vt_col0 = 2 * H;
         q.vt_ld = vt_ld;
-        if (lin("80", q, "enc_gemm_qkv") != 0) return 1;
-      } else if (gemm(h, L.w_qkv, a8 ? L.w_qkv8 : nullptr, L.s_qkv, L.b_qkv, qkv, nullptr, 3 * H, H, 0,
-               "enc_gemm_qkv", vt) != 0)
+        if (lin8(q, 0, "enc_gemm_qkv") != 0) return 1;
+      } else if (gemm(h, L.w_qkv, a8 ? L.w_qkv8 : nullptr, L.s_qkv, L.b_qkv, qkv, nullptr, 3 * H, H,
+                      0, "enc_gemm_qkv", vt) != 0) {
         return 1;
+      }
       const double log2e = 1.4426950408889634;
       EncAttnArgs at{qkv, vt, ctx, seq_off, seq_cnt, seq_q, batch, nh, H, tokens, vt_ld,
                      (float)(scaled_scores ? log2e / std::sqrt((double)hd) : log2e), status + 1,
@@ -510,36 +537,19 @@ struct EosHipEncoder {
                      err) != 0)
         return 1;
       if (small) {
-        EncLinArgs o{};
-        o.x = ctx;
-        o.w = L.w_of;
-        o.s = L.s_o;
-        o.b = L.b_o;
-        o.res = prev == nullptr ? h : hb;
-        o.out = h;
-        o.n = o.k = H;
         EncLinArgs u{};
         u.x = h;
         u.gamma = L.g1;
         u.beta = L.be1;
-        u.ln_out = ctx;
+        u.ln_out = ctx;  // free once the O projection has read it
         u.w = L.w_1f;
         u.s = L.s_1;
         u.b = L.b_1;
         u.out = mid;
         u.n = F;
-        EncLinArgs dn{};
-        dn.x = mid;
-        dn.w = L.w_2f;
-        dn.s = L.s_2;
-        dn.b = L.b_2;
-        dn.res = ctx;
-        dn.out = h;
-        dn.n = H;
-        dn.k = F;
-        if (lin("16", o, "enc_gemm_o") != 0 ||
-            lin(desc.gelu == 1 ? "81" : "82", u, "enc_gemm_ffn_up") != 0 ||
-            lin("16", dn, "enc_gemm_ffn_down") != 0)
+        if (project(ctx, L.w_of, L.w_o, L.s_o, L.b_o, prev == nullptr ? h : hb, H, "enc_gemm_o") != 0 ||
+            lin8(u, desc.gelu, "enc_gemm_ffn_up") != 0 ||
+            project(mid, L.w_2f, L.w_2, L.s_2, L.b_2, ctx, F, "enc_gemm_ffn_down") != 0)
           return 1;
         prev = &L;
         continue;
@@ -578,11 +588,11 @@ struct EosHipEncoder {
           return 1;
         continue;
       }
-      if (gemm(ctx, L.w_o, nullptr, L.s_o, L.b_o, h, h, H, H, 3, "enc_gemm_o") != 0 ||
+      if (project(ctx, L.w_of, L.w_o, L.s_o, L.b_o, h, H, "enc_gemm_o") != 0 ||
           layer_norm(L.g1, L.be1) != 0 ||
           gemm(h, L.w_1, a8 ? L.w_18 : nullptr, L.s_1, L.b_1, mid, nullptr, F, H, desc.gelu,
                "enc_gemm_ffn_up") != 0 ||
-          gemm(mid, L.w_2, nullptr, L.s_2, L.b_2, h, h, H, F, 3, "enc_gemm_ffn_down") != 0 ||
+          project(mid, L.w_2f, L.w_2, L.s_2, L.b_2, h, F, "enc_gemm_ffn_down") != 0 ||
           layer_norm(L.g2, L.be2) != 0)
         return 1;
     }

@@ -1473,8 +1473,6 @@ EOS_TAIL_KERNEL(2, 512, 1)
 EOS_TAIL_KERNEL(2, 512, 2)
 EOS_TAIL_KERNEL(1, 512, 1)
 EOS_TAIL_KERNEL(1, 512, 2)
-EOS_TAIL_KERNEL(1, 768, 1)
-EOS_TAIL_KERNEL(1, 768, 2)
 #undef EOS_TAIL_KERNEL
 
 // ------------------------------------------------- small-batch linear layers
@@ -1482,17 +1480,19 @@ EOS_TAIL_KERNEL(1, 768, 2)
 namespace {
 
 // The BERT layer for batches whose row blocks cannot fill the chip as fused
-// tails (a 96-row tail block runs a whole layer's weights on one CU: 24 rows
-// at H 384, 61 us per layer on one block): every linear layer spread over row
-// tiles x column blocks, the LayerNorms in the prologue of the layer that
-// reads them. The sums run in the same K order on the same instructions, and
-// every value is rounded where the tail and the wide GEMMs round it, so the
-// embeddings do not depend on which path a batch takes.
+// tails (a tail block runs a whole layer's weights on one CU: 61 us per layer
+// for 24 rows at H 384): every linear layer spread over row tiles x column
+// blocks, the LayerNorms in the prologue of the layer that reads them. The
+// sums run in the same K order on the same instructions, and every value is
+// rounded where the tail and the wide GEMMs round it, so the embeddings do
+// not depend on which path a batch takes.
 //
 // Workgroup: 32 rows x 256 columns, wavefront w the columns [32 w, + 32) of
 // the block. All of a wavefront's weights (H / 32 KB) are requested before the
 // LayerNorm, which 8 wavefronts run on 4 rows each. Every column block of a
-// row tile repeats the LayerNorm; the first writes its rows out.
+// row tile repeats the LayerNorm; the first writes its rows out. Bound by
+// latency: one round trip for weights and rows, the LayerNorm's reductions,
+// H / 32 MFMAs (24 rows, H 384: QKV 5.9, FFN up 6.8 us).
 // EPI 0: QKV, 1: erf GELU, 2: tanh GELU.
 template <int H, int EPI>
 struct Lin8 {
@@ -1591,97 +1591,111 @@ struct Lin8 {
   }
 };
 
-// The O and FFN-down projections of small batches: 64 rows x 128 columns per
-// workgroup, wavefront w the columns [32 w, + 32), K in chunks of 128 through
-// two LDS stages (one barrier per chunk), weights eight K steps ahead.
+// The O and FFN-down projections of small batches: 32 RT rows x 128 columns
+// per workgroup, wavefront w the columns [32 w, + 32). A stage holds 512 / RT K
+// values of the rows (one barrier per stage, the next one's loads in flight
+// meanwhile), weights come 16 K steps ahead: with few workgroups the time is
+// one memory round trip per stage plus the MFMA chain (24 rows, H 384, K 1536:
+// 8.5 us with 32-row workgroups, 12.3 with 64; 128 K values per stage with
+// weights 8 steps ahead 18).
 // out = acc s + b + res, rounded once (out may alias res).
-constexpr int kLinK = 128;
-struct Lin16Lds {
-  uint16_t a[2][64 * (kLinK + 8)];
-};
-EOS_DEV void lin16_body(const EncLinArgs& a, Lin16Lds& s) {
-  constexpr int BM = 64, RT = 2, AS = kLinK + 8, PER = BM * kLinK / 8 / 256;
-  const int ncb = a.n / 128;
-  const int m0 = (int)(blockIdx.x / ncb) * BM, n0 = (blockIdx.x % ncb) * 128;
-  const int rows = *a.rows;
-  if (m0 >= rows) return;
-  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, l32 = lane & 31;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nw = n0 + 32 * wave, nk = a.k / kLinK;
-  const v8h* wsrc = reinterpret_cast<const v8h*>(a.w) + (size_t)(nw / 32) * (a.k / 16) * 64 + lane;
-  v8h wq[8];
-#pragma unroll
-  for (int p = 0; p < 8; ++p) wq[p] = wsrc[64 * p];
-  v4i st[PER];
-  auto load = [&](int c) {
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int i = tid + 256 * u, r = i / (kLinK / 8), k8 = i % (kLinK / 8);
-      st[u] = *reinterpret_cast<const v4i*>(a.x + (size_t)min(m0 + r, a.max_rows - 1) * a.k +
-                                            kLinK * c + 8 * k8);
-    }
+template <int RT>
+struct Lin16 {
+  static constexpr int BM = 32 * RT, KC = 512 / RT, AS = KC + 8, PF = 16;
+  static constexpr int PER = BM * KC / 8 / 256;  // 16-byte loads per thread per stage
+  struct Lds {
+    uint16_t a[2][BM * AS];
   };
-  auto store = [&](int b) {
+  EOS_DEV static void run(const EncLinArgs& a, Lds& s) {
+    const int ncb = a.n / 128;
+    const int m0 = (int)(blockIdx.x / ncb) * BM, n0 = (blockIdx.x % ncb) * 128;
+    const int rows = *a.rows;
+    if (m0 >= rows) return;
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, l32 = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nw = n0 + 32 * wave, ksn = a.k / 16, nst = (a.k + KC - 1) / KC;
+    const v8h* wsrc = reinterpret_cast<const v8h*>(a.w) + (size_t)(nw / 32) * ksn * 64 + lane;
+    v4i st[PER];
+    // (K past the end: the last values again, never multiplied)
+    auto load = [&](int c) {
 #pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int i = tid + 256 * u, r = i / (kLinK / 8), k8 = i % (kLinK / 8);
-      *reinterpret_cast<v4i*>(&s.a[b][r * AS + 8 * k8]) = st[u];
-    }
-  };
-  load(0);
-  // The residual is requested with the first chunk.
-  v4h res[RT][4];
+      for (int u = 0; u < PER; ++u) {
+        const int i = tid + 256 * u, r = i / (KC / 8), k = KC * c + 8 * (i % (KC / 8));
+        st[u] = *reinterpret_cast<const v4i*>(a.x + (size_t)min(m0 + r, a.max_rows - 1) * a.k +
+                                              min(k, a.k - 8));
+      }
+    };
+    auto store = [&](int b) {
 #pragma unroll
-  for (int i = 0; i < RT; ++i)
+      for (int u = 0; u < PER; ++u) {
+        const int i = tid + 256 * u, r = i / (KC / 8), k8 = i % (KC / 8);
+        *reinterpret_cast<v4i*>(&s.a[b][r * AS + 8 * k8]) = st[u];
+      }
+    };
+    load(0);
+    v8h wq[PF];
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-      res[i][q] = *reinterpret_cast<const v4h*>(
-          a.res + (size_t)min(m0 + 32 * i + l32, a.max_rows - 1) * a.n + nw + 8 * q + 4 * g);
-  store(0);
-  load(min(1, nk - 1));
-  __syncthreads();
-  v16f acc[RT];
-#pragma unroll
-  for (int i = 0; i < RT; ++i) acc[i] = v16f{0};
-  for (int c = 0; c < nk; ++c) {
-    const uint16_t* A = s.a[c & 1];
-    const int nx = min(c + 1, nk - 1) * 8;  // the next chunk's first K step
-#pragma unroll
-    for (int kk = 0; kk < 8; ++kk) {
-      v8h bf[RT];
-#pragma unroll
-      for (int i = 0; i < RT; ++i)
-        bf[i] = *reinterpret_cast<const v8h*>(&A[(32 * i + l32) * AS + 16 * kk + 8 * g]);
-      const v8h af = wq[kk];
-      wq[kk] = wsrc[64 * (size_t)(nx + kk)];
-#pragma unroll
-      for (int i = 0; i < RT; ++i)
-        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, bf[i], acc[i], 0, 0, 0);
-    }
-    store((c + 1) & 1);
-    load(min(c + 2, nk - 1));
+    for (int p = 0; p < PF; ++p) wq[p] = wsrc[64 * min(p, ksn - 1)];
+    store(0);
+    load(1);
     __syncthreads();
-  }
+    v16f acc[RT];
 #pragma unroll
-  for (int i = 0; i < RT; ++i) {
-    const int row = m0 + 32 * i + l32;
-    if (row >= rows) continue;
+    for (int i = 0; i < RT; ++i) acc[i] = v16f{0};
+    for (int c = 0; c < nst; ++c) {
+      // 8 K steps (K is a multiple of 128) at a time; a stage has a whole
+      // number of them, and every second one starts at ring slot 0.
+      const int sub = min(KC, a.k - KC * c) / 128;
+      const uint16_t* A = s.a[c & 1] + l32 * AS + 8 * g;
+      auto eight = [&](int h, auto half_c) {
+        constexpr int kHalf = decltype(half_c)::value;
+        const int ks0 = (KC / 16) * c + 8 * h;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int n = nw + 8 * q + 4 * g;
-      const float4 sc = *reinterpret_cast<const float4*>(a.s + n);
-      const float4 bi = *reinterpret_cast<const float4*>(a.b + n);
-      float v[4] = {__builtin_fmaf(acc[i][4 * q], sc.x, bi.x),
-                    __builtin_fmaf(acc[i][4 * q + 1], sc.y, bi.y),
-                    __builtin_fmaf(acc[i][4 * q + 2], sc.z, bi.z),
-                    __builtin_fmaf(acc[i][4 * q + 3], sc.w, bi.w)};
-      v4h o;
+        for (int kk = 0; kk < 8; ++kk) {
+          v8h bf[RT];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) o[t] = (_Float16)(v[t] + (float)res[i][q][t]);
-      *reinterpret_cast<v4h*>(a.out + (size_t)row * a.n + n) = o;
+          for (int i = 0; i < RT; ++i)
+            bf[i] = *reinterpret_cast<const v8h*>(&A[32 * i * AS + 128 * h + 16 * kk]);
+          const v8h af = wq[8 * kHalf + kk];
+          wq[8 * kHalf + kk] = wsrc[64 * min(ks0 + kk + PF, ksn - 1)];
+#pragma unroll
+          for (int i = 0; i < RT; ++i)
+            acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, bf[i], acc[i], 0, 0, 0);
+        }
+      };
+      for (int h = 0; h < sub; h += 2) {
+        eight(h, std::integral_constant<int, 0>{});
+        if (h + 1 < sub) eight(h + 1, std::integral_constant<int, 1>{});
+      }
+      store((c + 1) & 1);
+      load(c + 2);
+      __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+      const int row = m0 + 32 * i + l32;
+      if (row >= rows) continue;
+      v4h res[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        res[q] = *reinterpret_cast<const v4h*>(a.res + (size_t)row * a.n + nw + 8 * q + 4 * g);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int n = nw + 8 * q + 4 * g;
+        const float4 sc = *reinterpret_cast<const float4*>(a.s + n);
+        const float4 bi = *reinterpret_cast<const float4*>(a.b + n);
+        float v[4] = {__builtin_fmaf(acc[i][4 * q], sc.x, bi.x),
+                      __builtin_fmaf(acc[i][4 * q + 1], sc.y, bi.y),
+                      __builtin_fmaf(acc[i][4 * q + 2], sc.z, bi.z),
+                      __builtin_fmaf(acc[i][4 * q + 3], sc.w, bi.w)};
+        v4h o;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) o[t] = (_Float16)(v[t] + (float)res[q][t]);
+        *reinterpret_cast<v4h*>(a.out + (size_t)row * a.n + n) = o;
+      }
     }
   }
-}
+};
 
 }  // namespace
 
@@ -1698,10 +1712,14 @@ EOS_LIN8_KERNELS(512)
 EOS_LIN8_KERNELS(768)
 #undef EOS_LIN8_KERNELS
 #undef EOS_LIN8_KERNEL
-extern "C" __global__ __launch_bounds__(256) void eos_enc_lin16(EncLinArgs a) {
-  __shared__ __attribute__((aligned(16))) Lin16Lds lds;
-  lin16_body(a, lds);
-}
+#define EOS_LIN16_KERNEL(RT)                                                              \
+  extern "C" __global__ __launch_bounds__(256) void eos_enc_lin16_r##RT(EncLinArgs a) {   \
+    __shared__ __attribute__((aligned(16))) Lin16<RT>::Lds lds;                           \
+    Lin16<RT>::run(a, lds);                                                               \
+  }
+EOS_LIN16_KERNEL(1)
+EOS_LIN16_KERNEL(2)
+#undef EOS_LIN16_KERNEL
 
 // --------------------------------------------------------------- attention
 

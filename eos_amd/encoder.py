@@ -256,8 +256,8 @@ class Encoder:
         return st.value
 
     def set_fused_tail(self, fused: bool) -> None:
-        """BERT family at hidden 384 / 512 / 768: run the layer tail as one
-        fused kernel (default) or as the unfused GEMM + LayerNorm launches."""
+        """BERT family: the fused layer paths (default) or GEMM + LayerNorm
+        launches throughout."""
         _lib.call("eoship_encoder_set_fused_tail", self.rt.handle, self.handle, C.c_int32(int(fused)))
 
     def set_pooling(self, pooling: str) -> None:

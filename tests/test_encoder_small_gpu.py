@@ -1,8 +1,9 @@
 """Small batches of the BERT family (eos_enc_lin8 / eos_enc_lin16 launches):
 bit-identical to the unfused launches at the edges of their tiles (32 and 64
 rows, 256 and 128 columns) for every width, both GELUs, both poolings and
-token types, and within the contract of the CPU oracle; and bit-identical to the same sequence in a batch large enough for the wide GEMM
-and fused tail."""
+token types, and within the contract of the CPU oracle; and bit-identical to
+the same sequence in batches that take the other paths (LayerNorm launches
+with the wide GEMM, 64-row tiles, the fused tail)."""
 import numpy as np
 import pytest
 
@@ -46,8 +47,9 @@ def test_small_batch_matches_oracle(rt, hidden, heads, inter, lens, gelu, poolin
     enc.release()
 
 
-@pytest.mark.parametrize("hidden,heads,batch", [(384, 12, 24), (512, 8, 22), (768, 12, 20),
-                                                (256, 8, 52)])
+@pytest.mark.parametrize("hidden,heads,batch", [(384, 12, 12), (384, 12, 32), (512, 8, 8),
+                                                (512, 8, 32), (768, 12, 6), (768, 12, 24),
+                                                (256, 8, 36)])
 def test_small_and_large_batches_agree_bit_for_bit(rt, hidden, heads, batch):
     from eos_amd.encoder import Encoder
     print(f"[case] small against large batch H={hidden}", flush=True)
