@@ -386,11 +386,11 @@ struct EosHipTQ {
 
   // Prepares nq queries of tq tokens (source rows [nq * tq][d]) at once: query
   // g is the 32-column group g (tokens past tq are zero columns), rounded up
-  // to whole passes of maxsim_nqg() groups.
+  // to whole passes of the kernels that read them.
   // With `bounds` also each column's ||lo||_2 (ms_lonorm) for the high-half
   // bound filter.
   int maxsim_prepare(const float* d_src, int nq, int tq, char** err, bool bounds = false) {
-    const int per = maxsim_nqg();
+    const int per = bounds && maxsim_wide(nq) ? 8 : maxsim_nqg();
     const int groups = (nq + per - 1) / per * per;
     const size_t cols = (size_t)groups * 32;
     if (ensure(reinterpret_cast<void**>(&ms_bfrag), &ms_bfrag_bytes, (size_t)ks * 2 * groups * 64 * 16,
@@ -431,10 +431,22 @@ struct EosHipTQ {
     return m;
   }
 
+  // The bound filter over 8 groups a pass: at short K its per-tile work
+  // (decode, norms) is a third of the instructions at 4 groups (32 x 32
+  // tokens over 12.8 million rows of dim 128: 2076 -> 1800 us). Not where the
+  // rounding up to 8 would add a group pass to every three or fewer.
+  bool maxsim_wide(int groups) const {
+    const int p4 = (groups + 3) / 4;
+    return ks <= 4 && p4 > 1 && (p4 % 2 == 0 || p4 >= 5);
+  }
+
   // Launches MaxSim kernel `hi` (bound filter) or exact over `docs` documents
-  // per pass, for m.groups groups in passes of maxsim_nqg().
+  // per pass, for m.groups groups; listed documents are scored one group a
+  // pass (each group has its own list).
   int maxsim_launch(TqMaxsimArgs* m, bool hi, int64_t docs, const char* label, char** err) {
-    const int nqg = maxsim_nqg();
+    int nqg = maxsim_nqg();
+    if (hi && maxsim_wide(m->groups)) nqg = 8;
+    if (m->doc_list != nullptr) nqg = 1;
     char name[64];
     snprintf(name, sizeof(name), "eos_tq_maxsim_b%d_k%d_g%d%s", bits, ks, nqg, hi ? "_h" : "");
     // As many resident workgroups as the kernel's registers allow (three
@@ -1210,41 +1222,54 @@ int rank_rows(EosHipRuntime* rt, const float* d_rows, int rows, int64_t n, int k
 // kMsMaxK, ndocs >= kMsMinDocs), all passes in each launch:
 //  1. exact scores of every stride-th document (at most kMsSampleDocs), and
 //     per query tau = the r-th best of them, r chosen so that about
-//     min(3 kk, kMsCap / 8) documents of the corpus are expected above it;
+//     min(3 kk, kMsTarget) documents of the corpus are expected above it;
 //  2. the high-half bound filter over every document: a document is listed
-//     for its pass when its score bound reaches tau of one of the pass's
-//     queries (a bound >= the exact score, so every document scoring >= tau
-//     is listed);
-//  3. exact scores of the listed documents as rank keys (0 below tau), and
-//     per query the top kk of them (eos_tq_finalize): final when at least kk
-//     listed documents score >= tau, since every unlisted one scores below;
-//  4. otherwise (too few, or the list overflowed kMsCap) the query is
-//     flagged and its row recomputed exhaustively, gated on the device.
+//     for a query when its score bound reaches the query's tau (a bound >=
+//     the exact score, so every document scoring >= tau is listed);
+//  3. exact scores of the listed documents, the rank keys of those >= tau
+//     kept per query, and the top kk of them (eos_tq_finalize): final when
+//     there are at least kk, since every unlisted document scores below tau;
+//  4. otherwise (too few, the list overflowed kMsList or the kept keys
+//     kMsCap) the query is flagged and its row recomputed exhaustively, gated
+//     on the device. The list holds the documents that only the bound lets
+//     through too (at 100,000 documents x 128 rows of dim 128 about 2,000 for
+//     430 above tau), so it has twice the keys' capacity.
 // Results equal the exhaustive path's: the same exact scores, ranked by
 // (score desc, document index asc).
 constexpr int kMsCap = 8192;
+constexpr int kMsList = 16384;
+constexpr int kMsTarget = 1024;
 constexpr int kMsSampleDocs = 2048;
 constexpr int kMsMinDocs = 16384;
 constexpr int kMsMaxK = 512;
 int maxsim_filtered(EosHipRuntime* rt, EosHipTQ* tq, int doc_len, int64_t ndocs, int cq, int kk,
                     int64_t* d_ids, float* d_scores, char** err) {
-  const int per = tq->maxsim_nqg();
-  const int npass = (cq + per - 1) / per;
   const int64_t stride = std::max<int64_t>(16, (ndocs + kMsSampleDocs - 1) / kMsSampleDocs);
   const int64_t ns = (ndocs + stride - 1) / stride;
-  const double target = std::min<double>(3.0 * kk, kMsCap / 8.0);
+  const double target = std::min<double>(3.0 * kk, kMsTarget);
   int64_t r = (int64_t)std::ceil(target * (double)ns / (double)ndocs);
+  // Fewer than kk documents score >= tau when r or more of the sample are
+  // among the best kk, a Poisson count of mean x: r of at least x + 3 sqrt(x)
+  // + 2 makes that about one query in 3,000 (at 100,000 documents and k = 100
+  // 3 kk alone, r = 7, one in 200: with 32 queries every seventh call paid an
+  // exhaustive pass, 1.5 ms, where two more list entries in seven cost 40
+  // us), unless so many documents above tau would crowd the kept keys.
+  const double x = (double)kk * (double)ns / (double)ndocs;
+  const int64_t safe = (int64_t)std::ceil(x + 3.0 * std::sqrt(x) + 2.0);
+  const int64_t room = (int64_t)((double)(kMsCap / 2) * (double)ns / (double)ndocs);
+  r = std::max(r, std::min(safe, room));
   r = std::max<int64_t>(1, std::min<int64_t>(r, ns));
-  // workspace: samples [cq][ns] f32, tau [cq], list [npass][cap] u32, list
-  // counts [npass], rank keys [cq][cap] u64, key counts [cq], status [cq]
+  // workspace: samples [cq][ns] f32, tau [cq], lists [cq][kMsList] u32, list
+  // counts [cq] and key counts [cq] (cleared together), rank keys
+  // [cq][kMsCap] u64, status [cq]
   auto al = [](size_t b) { return (b + 255) / 256 * 256; };
   const size_t o_samp = 0;
   const size_t o_tau = o_samp + al((size_t)cq * ns * 4);
   const size_t o_list = o_tau + al((size_t)cq * 4);
-  const size_t o_lcnt = o_list + al((size_t)npass * kMsCap * 4);
-  const size_t o_cand = o_lcnt + al((size_t)npass * 4);
-  const size_t o_ccnt = o_cand + al((size_t)cq * kMsCap * 8);
-  const size_t o_stat = o_ccnt + al((size_t)cq * 4);
+  const size_t o_lcnt = o_list + al((size_t)cq * kMsList * 4);
+  const size_t o_ccnt = o_lcnt + (size_t)cq * 4;
+  const size_t o_cand = o_lcnt + al((size_t)cq * 8);
+  const size_t o_stat = o_cand + al((size_t)cq * kMsCap * 8);
   const size_t total = o_stat + al((size_t)cq * 4);
   if (tq->ensure(&tq->ms_ws, &tq->ms_ws_bytes, total, err) != 0) return 1;
   char* w = static_cast<char*>(tq->ms_ws);
@@ -1274,7 +1299,7 @@ int maxsim_filtered(EosHipRuntime* rt, EosHipTQ* tq, int doc_len, int64_t ndocs,
   if (rt->launch("eos_tq_threshold", dim3((unsigned)cq), dim3(256), 0, &sel, err, "tq_maxsim_threshold") != 0)
     return 1;
   // 2. bound filter
-  hipError_t e = hipMemsetAsync(lcnt, 0, (size_t)npass * 4, rt->stream);
+  hipError_t e = hipMemsetAsync(lcnt, 0, (size_t)cq * 8, rt->stream);
   if (e != hipSuccess) return hip_err(err, "hipMemsetAsync(list counts)", e);
   m = tq->maxsim_args(0, cq, doc_len);
   m.doc_begin = 0;
@@ -1284,18 +1309,19 @@ int maxsim_filtered(EosHipRuntime* rt, EosHipTQ* tq, int doc_len, int64_t ndocs,
   m.tile_cn = tq->tile_cn;
   m.list = list;
   m.list_count = lcnt;
-  m.list_cap = kMsCap;
+  m.list_cap = kMsList;
   if (tq->maxsim_launch(&m, true, ndocs, "tq_maxsim_filter", err) != 0) return 1;
   // 3. exact scores of the listed documents, then the top kk of each query
   m = tq->maxsim_args(0, cq, doc_len);
-  m.ndocs = kMsCap;
+  m.ndocs = std::min<int64_t>(kMsList, ndocs);
   m.doc_list = list;
   m.list_count = lcnt;
-  m.list_cap = kMsCap;
+  m.list_cap = kMsList;
+  m.cand_cap = kMsCap;
   m.cand = cand;
   m.cand_count = ccnt;
   m.tau = tau;
-  if (tq->maxsim_launch(&m, false, kMsCap, "tq_maxsim_rescore", err) != 0) return 1;
+  if (tq->maxsim_launch(&m, false, m.ndocs, "tq_maxsim_rescore", err) != 0) return 1;
   TqFinalizeArgs f;
   memset(&f, 0, sizeof(f));
   f.cand = cand;

@@ -111,8 +111,10 @@ struct TqMaxsimArgs {
   // launch (alpha, out, tau, gate, lonorm and the doc lists offset by it).
   // Document i of a pass is doc_begin + i * doc_stride (doc_stride 0 = 1),
   // or, with doc_list, doc_list[p * list_cap + i] for i < min(count, cap),
-  // count = list_count[p]; in that mode the exact scores leave as rank keys
-  // cand[group][i] (0 when below tau[group]) with cand_count[group] = count.
+  // count = list_count[p]; in that mode the exact scores >= tau[group] are
+  // appended as rank keys to cand[group * cand_cap ..], counted in
+  // cand_count[group] (cleared by the caller; entries past cand_cap dropped),
+  // which an overflowed list raises by 2^30.
   long long doc_stride;
   const uint32_t* doc_list;
   unsigned long long* cand;
@@ -120,13 +122,13 @@ struct TqMaxsimArgs {
   const float* tau;        // [groups]
   const int* gate;         // or NULL: a pass runs only if a live group's gate is set
   // High-half bound filter (the _h kernels): documents whose score bound
-  // reaches tau of some live group of the pass are appended to
-  // list[p * list_cap ..] (count list_count[p], entries past cap dropped).
+  // reaches tau of a live group are appended to list[group * list_cap ..]
+  // (count list_count[group], entries past cap dropped).
   const float* lonorm;     // [32 * groups] ||lo||_2 of each column, rounded up
   const float* tile_cn;    // [2 * tiles] largest ||C[codes]||_2 of the tile, largest Norm
   uint32_t* list;
   uint32_t* list_count;
-  int list_cap;
+  int list_cap, cand_cap;
 };
 
 // Parent (multivector) aggregation over child scores: parent p owns children

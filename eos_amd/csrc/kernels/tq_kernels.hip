@@ -2139,6 +2139,28 @@ EOS_DEV void maxsim_bound(float& my, const v16i& hi, float lb, const float (&nrm
   for (int i = 0; i < 16; ++i) my = fmaxf(my, __builtin_fmaf((float)hi[i], 256.0f, lb) * nrm[i]);
 }
 
+// The same bound for D <= 256 (KS <= 8), one fma and half a maximum per
+// element instead of a conversion, an fma, a product and a maximum: at short
+// K the vector unit, not the matrix unit, bounds the filter. The MFMAs start
+// from kBoundMagic + L, L = ceil(lb / 256) + 1, so a result's bits are the
+// float M + D_hi + L, M = 3 2^22, exactly: |D_hi| <= 256 * 127 * 128 and L <=
+// 16,258 stay inside the 2^22 on either side of M. With nc = fl(-M n), y =
+// fma(M + D_hi + L, n, nc) is n (D_hi + L) less at most 0.75 n (the rounding
+// of nc, covered by L's + 1) and one rounding, so 256 alpha max(y, 0) (1 +
+// 2^-20) is at least every exact score as long as M n does not overflow (the
+// caller lists a document whose largest Norm is 2^100 or more).
+constexpr int kBoundMagic = 0x4b400000;  // 12582912.0f = 3 * 2^22
+EOS_DEV void maxsim_bound_short(float& my, const v16i& acc, const float (&nrm)[16],
+                                const float (&nc)[16]) {
+#pragma unroll
+  for (int i = 0; i < 16; i += 2) {
+    const float y0 = __builtin_fmaf(__int_as_float(acc[i]), nrm[i], nc[i]);
+    const float y1 = __builtin_fmaf(__int_as_float(acc[i + 1]), nrm[i + 1], nc[i + 1]);
+    // One instruction for fmaxf(my, fmaxf(y0, y1)).
+    asm("v_max3_f32 %0, %1, %2, %0" : "+v"(my) : "v"(y0), "v"(y1));
+  }
+}
+
 // Register stages of the MaxSim tile ring: as many as fit beside the
 // accumulators in the 168 registers of three waves per SIMD.
 template <bool HI>
@@ -2186,7 +2208,7 @@ EOS_DEV float ms_token_sum(float v, int lane) {
 
 // MaxSim of documents against NQG query groups (32 token columns each) per
 // pass; HI: the high-half bound filter (half the MFMAs) that lists the
-// documents whose score bound reaches some group's tau.
+// documents whose score bound reaches a group's tau, one list per group.
 template <int BITS, int KS, int NQG, bool HI>
 EOS_DEV void tq_maxsim_body(const TqMaxsimArgs& a) {
   constexpr int NCB = 2 * NQG;
@@ -2194,6 +2216,7 @@ EOS_DEV void tq_maxsim_body(const TqMaxsimArgs& a) {
   constexpr int SPL = 8 / BITS;
   constexpr int NLOAD = (KS + SPL - 1) / SPL;
   constexpr int NWV = kScanThreads / 64;
+  constexpr bool SHORT = HI && KS <= 8;  // the bound by maxsim_bound_short
   __shared__ v4i sb[KS * NCBU * 64];
   __shared__ float4 nstage[NWV][8];
   const int goff = blockIdx.y * NQG;          // first query group of this pass
@@ -2209,7 +2232,10 @@ EOS_DEV void tq_maxsim_body(const TqMaxsimArgs& a) {
   if (dlist != nullptr) {
     const uint32_t c = a.list_count[blockIdx.y];
     ndocs = c < (uint32_t)a.list_cap ? (long long)c : (long long)a.list_cap;
-    if (blockIdx.x == 0 && threadIdx.x < (unsigned)gl) a.cand_count[goff + threadIdx.x] = c;
+    // An overflowed list: more candidates than any capacity, for finalize.
+    if (c > (uint32_t)a.list_cap && blockIdx.x == 0 && threadIdx.x < (unsigned)gl)
+      atomicAdd(&a.cand_count[goff + threadIdx.x], 1u << 30);
+    if ((long long)blockIdx.x * NWV >= ndocs) return;
   }
   {
     // The pass's column blocks of each K step (HI: the high blocks only;
@@ -2314,18 +2340,39 @@ EOS_DEV void tq_maxsim_body(const TqMaxsimArgs& a) {
   long long doc = doc0;
   int t = 0;
   float mx[NQG];
+  // SHORT: the MFMAs' start value. L takes the largest lonorm of the lane's
+  // columns and the largest code-norm bound of the tiles so far, so one set
+  // of registers serves every group and is rarely rewritten.
+  v16i start = {0};
+  float start_cn = -1.0f, lo_max = 0.0f;
+  bool wide = false;  // a Norm of the document is out of maxsim_bound_short's range
+#pragma unroll
+  for (int g = 0; g < NQG; ++g) lo_max = fmaxf(lo_max, lo_r[g]);
   auto process = [&](const Stage& st) {
     if (t == 0) {
 #pragma unroll
       for (int g = 0; g < NQG; ++g) mx[g] = -__builtin_inff();
+      wide = false;
     }
     int boff = lane;
     asm volatile("" : "+v"(boff));
     float lb[NQG];
     if constexpr (HI) {
       const float cn = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(st.nv), 32));
+      if constexpr (SHORT) {
+        const float nm = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(st.nv), 33));
+        wide |= !(nm < 0x1p100f);
+        if (cn > start_cn) {
+          start_cn = cn;
+          const float l = (lo_max * cn) * (1.0000002f / 256.0f);
+          const int v = kBoundMagic + (int)__builtin_ceilf(l) + 1;
 #pragma unroll
-      for (int g = 0; g < NQG; ++g) lb[g] = (lo_r[g] * cn) * 1.0000002f;  // >= lonorm * cn
+          for (int i = 0; i < 16; ++i) start[i] = v;
+        }
+      } else {
+#pragma unroll
+        for (int g = 0; g < NQG; ++g) lb[g] = (lo_r[g] * cn) * 1.0000002f;  // >= lonorm * cn
+      }
     }
     // Row r's norm sits at float r of the wave's slot; lane l needs rows
     // 8 i4 + 4 (l / 32) + {0..3}. LDS operations of one wave complete in
@@ -2342,11 +2389,18 @@ EOS_DEV void tq_maxsim_body(const TqMaxsimArgs& a) {
       nrm[4 * i4 + 3] = v.w;
     }
     __builtin_amdgcn_wave_barrier();
+    float nc[16];
+    if constexpr (SHORT) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) nc[i] = nrm[i] * -12582912.0f;
+    }
     // The score's "+ 0.0f" (-0 -> +0) commutes with the maximum (fmaxf
     // treats the zeros as equal), so it is applied once to the token max.
     v16i acc[NCB];
     auto epi = [&](int g) {
-      if constexpr (HI)
+      if constexpr (SHORT)
+        maxsim_bound_short(mx[g], acc[g], nrm, nc);
+      else if constexpr (HI)
         maxsim_bound(mx[g], acc[g], lb[g], nrm);
       else
         maxsim_epilogue(mx[g], acc[2 * g], acc[2 * g + 1], al[g], nrm);
@@ -2369,7 +2423,7 @@ EOS_DEV void tq_maxsim_body(const TqMaxsimArgs& a) {
       for (int g = 0; g <= NQG; ++g) {
         if (g < NQG) {
           if constexpr (HI) {
-            acc[g] = v16i{0};
+            acc[g] = start;
 #pragma unroll
             for (int s = 0; s < KS; ++s) {
               const v4i bh = sb[(s * NCBU + g) * 64 + boff];
@@ -2415,30 +2469,33 @@ EOS_DEV void tq_maxsim_body(const TqMaxsimArgs& a) {
       for (int g = 0; g < NQG; ++g) epi(g);
     }
     if (t == tpd - 1) {
-      bool keep = false;
 #pragma unroll
       for (int g = 0; g < NQG; ++g) {
         float m0, m1;
         ms_halves(mx[g], m0, m1);
         float v = fmaxf(m0, m1);  // token max over the document
-        if constexpr (HI) v = (fmaxf(v, 0.0f) * al[g]) * 1.000001f;  // >= every exact token max
+        // HI: at least every exact token max (the last term covers results
+        // that round among the subnormals).
+        if constexpr (SHORT)
+          v = __builtin_fmaf(fmaxf(v, 0.0f) * (al[g] * 256.0f), 1.000001f, 1.2e-38f);
+        else if constexpr (HI)
+          v = (fmaxf(v, 0.0f) * al[g]) * 1.000001f;
         v = ms_token_sum(v + 0.0f, lane);
         if constexpr (HI) {
           // tau <= 0 (or NaN) cannot prune: every document is listed.
-          keep |= g < gl && (v >= ta_r[g] || !(ta_r[g] > 0.0f));
+          if (lane == 0 && g < gl && (v >= ta_r[g] || !(ta_r[g] > 0.0f) || wide)) {
+            const uint32_t pos = atomicAdd(&a.list_count[goff + g], 1u);
+            if (pos < (uint32_t)a.list_cap)
+              a.list[(size_t)(goff + g) * a.list_cap + pos] = (uint32_t)st.id;
+          }
         } else if (dlist != nullptr) {
-          if (lane == 0 && g < gl)
-            a.cand[(size_t)(goff + g) * a.list_cap + doc] =
-                v >= ta_r[g] ? rank_key(v, (uint32_t)st.id) : 0ull;
+          if (lane == 0 && g < gl && v >= ta_r[g]) {
+            const uint32_t pos = atomicAdd(&a.cand_count[goff + g], 1u);
+            if (pos < (uint32_t)a.cand_cap)
+              a.cand[(size_t)(goff + g) * a.cand_cap + pos] = rank_key(v, (uint32_t)st.id);
+          }
         } else {
           if (lane == 0 && g < gl) a.out[(size_t)(goff + g) * a.out_stride + doc] = v;
-        }
-      }
-      if constexpr (HI) {
-        if (lane == 0 && keep) {
-          const uint32_t pos = atomicAdd(&a.list_count[blockIdx.y], 1u);
-          if (pos < (uint32_t)a.list_cap)
-            a.list[(size_t)blockIdx.y * a.list_cap + pos] = (uint32_t)st.id;
         }
       }
     }
@@ -2482,6 +2539,47 @@ EOS_DEV void tq_maxsim_body(const TqMaxsimArgs& a) {
   void eos_tq_maxsim_b##BITS##_k##KS##_g##NQG##_h(TqMaxsimArgs a) {                          \
     tq_maxsim_body<BITS, KS, NQG, true>(a);                                                 \
   }
+
+// The bound filter over 8 query groups a pass. At 12.8 million rows of dim
+// 128 x 32 queries of 32 tokens: 2360 us with four vector instructions an
+// element, 2076 with maxsim_bound_short, 1765 with 8 groups a pass and a list
+// per group; the vector unit is busy 71 % of it (327 instructions a tile, 192
+// of them the bound), the matrix unit 51 %, at 1.8 GHz.
+#define EOS_TQ_MAXSIM_WIDE(BITS, KS)                                                        \
+  extern "C" __global__ __launch_bounds__(kScanThreads) __attribute__((amdgpu_waves_per_eu(3))) \
+  void eos_tq_maxsim_b##BITS##_k##KS##_g8_h(TqMaxsimArgs a) {                                \
+    tq_maxsim_body<BITS, KS, 8, true>(a);                                                \
+  }
+
+// The exact scores of one group's listed documents: scoring the union of
+// four groups' lists for all four cost 1.4x as much (same batch, 2,000
+// documents a list).
+#define EOS_TQ_MAXSIM_ONE(BITS, KS)                                                         \
+  extern "C" __global__ __launch_bounds__(kScanThreads) __attribute__((amdgpu_waves_per_eu(3))) \
+  void eos_tq_maxsim_b##BITS##_k##KS##_g1(TqMaxsimArgs a) {                                  \
+    tq_maxsim_body<BITS, KS, 1, false>(a);                                                  \
+  }
+
+EOS_TQ_MAXSIM_ONE(2, 1)
+EOS_TQ_MAXSIM_ONE(2, 2)
+EOS_TQ_MAXSIM_ONE(2, 4)
+EOS_TQ_MAXSIM_ONE(2, 8)
+EOS_TQ_MAXSIM_ONE(2, 12)
+EOS_TQ_MAXSIM_ONE(2, 16)
+EOS_TQ_MAXSIM_ONE(2, 24)
+EOS_TQ_MAXSIM_ONE(4, 1)
+EOS_TQ_MAXSIM_ONE(4, 2)
+EOS_TQ_MAXSIM_ONE(4, 4)
+EOS_TQ_MAXSIM_ONE(4, 8)
+EOS_TQ_MAXSIM_ONE(4, 12)
+EOS_TQ_MAXSIM_ONE(4, 16)
+EOS_TQ_MAXSIM_ONE(4, 24)
+EOS_TQ_MAXSIM_WIDE(2, 1)
+EOS_TQ_MAXSIM_WIDE(2, 2)
+EOS_TQ_MAXSIM_WIDE(2, 4)
+EOS_TQ_MAXSIM_WIDE(4, 1)
+EOS_TQ_MAXSIM_WIDE(4, 2)
+EOS_TQ_MAXSIM_WIDE(4, 4)
 
 EOS_TQ_MAXSIM(2, 1, 4)
 EOS_TQ_MAXSIM(2, 2, 4)
