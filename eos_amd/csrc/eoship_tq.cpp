@@ -2133,9 +2133,13 @@ int eoship_tq_ip_encode_device(EosHipRuntime* rt, const EosHipTQIPSpec* spec, co
   a.n = n;
   // 128 coordinates per tile row of the kernel (TJ); 32 vectors per workgroup
   // while their residuals fit the LDS beside the stages (d <= 512), else 16.
-  const int tj = (a.d + 127) / 128, per = tj <= 4 ? 32 : 16;
+  // Up to 16 vectors a CU a workgroup's own latency is the call: half the
+  // vectors and twice the load depth (us at n = 273: dim 150 35 -> 24, and
+  // n = 4,096: dim 384 62, where 6,000 in workgroups of 32 takes 100).
+  const bool small = n <= 16 * (int64_t)rt->compute_units;
+  const int tj = (a.d + 127) / 128, per = tj <= 4 && !small ? 32 : 16;
   char name[32];
-  snprintf(name, sizeof(name), "eos_tq_encode_ip_t%d", tj);
+  snprintf(name, sizeof(name), "eos_tq_encode_ip_%c%d", small ? 's' : 't', tj);
   return rt->launch(name, dim3((unsigned)((n + per - 1) / per)), dim3(512), 0, &a, err,
                     "tq_encode_ip");
 }

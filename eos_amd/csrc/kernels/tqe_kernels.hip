@@ -505,7 +505,10 @@ namespace {
 // of 8 vectors per CU); bound by the f64 matrix rate (118
 // GFLOP; dependent chains of this instruction reach 62 TFLOP/s at two
 // wavefronts per SIMD).
-template <int NV, int TJ>
+// P: steps (of four K values) a fragment load brings. Up to 16 vectors a CU
+// nothing hides a load's latency but the chain itself, so those calls take NV
+// = 1 and P = 8 (see the dispatch for both sides).
+template <int NV, int TJ, int P>
 struct EncodeIp {
   static constexpr int BV = 16 * NV, KC = 64, XST = KC + 4, RST = 128 * TJ + 4;
   static constexpr int kCodeRow = 64 * TJ;  // bytes: 8 TJ tiles x 16 codes of 4 bits
@@ -536,19 +539,19 @@ struct EncodeIp {
 #pragma unroll
         for (int t = 0; t < TJ; ++t) acc[n][t] = v4d{0.0, 0.0, 0.0, 0.0};
     };
-    // 16 K values (four steps) of the wavefront's rows of m [k][row].
-    auto load_m = [&](float (&f)[4][TJ], const float* m, int k0) {
+    // 4 P K values (P steps) of the wavefront's rows of m [k][row].
+    auto load_m = [&](float (&f)[P][TJ], const float* m, int k0) {
 #pragma unroll
-      for (int p = 0; p < 4; ++p) {
+      for (int p = 0; p < P; ++p) {
         const int k = k0 + 4 * p + lk;
         const float* row = m + (size_t)min(k, d - 1) * d;
 #pragma unroll
         for (int t = 0; t < TJ; ++t) f[p][t] = row[min(16 * (wave + 8 * t) + lr, d - 1)];
       }
     };
-    auto steps = [&](const float (&f)[4][TJ], int k0, auto&& right) {
+    auto steps = [&](const float (&f)[P][TJ], int k0, auto&& right) {
 #pragma unroll
-      for (int p = 0; p < 4; ++p) {
+      for (int p = 0; p < P; ++p) {
         const int k = k0 + 4 * p + lk;
         double b[NV];
 #pragma unroll
@@ -587,7 +590,7 @@ struct EncodeIp {
     load_x(1);
     clear();
     double ss = 0.0;
-    float fa[4][TJ], fb[4][TJ];
+    float fa[P][TJ], fb[P][TJ];
     const bool rot = a.rot_t != nullptr;
     if (rot) load_m(fa, a.rot_t, 0);
     lds_barrier();
@@ -596,11 +599,11 @@ struct EncodeIp {
       auto right = [&](int n, int k) { return (double)xc[(16 * n + lr) * XST + (k - KC * c)]; };
       if (rot) {
 #pragma unroll
-        for (int h = 0; h < KC / 32; ++h) {
-          load_m(fb, a.rot_t, KC * c + 32 * h + 16);
-          steps(fa, KC * c + 32 * h, right);
-          load_m(fa, a.rot_t, KC * c + 32 * h + 32);
-          steps(fb, KC * c + 32 * h + 16, right);
+        for (int h = 0; h < KC / (8 * P); ++h) {
+          load_m(fb, a.rot_t, KC * c + 8 * P * h + 4 * P);
+          steps(fa, KC * c + 8 * P * h, right);
+          load_m(fa, a.rot_t, KC * c + 8 * P * h + 8 * P);
+          steps(fb, KC * c + 8 * P * h + 4 * P, right);
         }
       }
       // The norms' chains (vector = thread).
@@ -697,11 +700,11 @@ struct EncodeIp {
     clear();
     auto right = [&](int n, int k) { return k < d ? s.rs[(16 * n + lr) * RST + k] : 0.0; };
     load_m(fa, a.qjl_t, 0);
-    for (int k0 = 0; k0 < d; k0 += 32) {
-      load_m(fb, a.qjl_t, k0 + 16);
+    for (int k0 = 0; k0 < d; k0 += 8 * P) {
+      load_m(fb, a.qjl_t, k0 + 4 * P);
       steps(fa, k0, right);
-      load_m(fa, a.qjl_t, k0 + 32);
-      if (k0 + 16 < d) steps(fb, k0 + 16, right);
+      load_m(fa, a.qjl_t, k0 + 8 * P);
+      if (k0 + 4 * P < d) steps(fb, k0 + 4 * P, right);
     }
 #pragma unroll
     for (int n = 0; n < NV; ++n)
@@ -743,17 +746,25 @@ struct EncodeIp {
 }  // namespace
 
 // 16 NV vectors per workgroup, up to 128 TJ coordinates.
-#define EOS_TQ_ENCODE_IP(NV, TJ)                                                        \
-  extern "C" __global__ __launch_bounds__(512) void eos_tq_encode_ip_t##TJ(TqIpArgs a) { \
-    __shared__ __attribute__((aligned(16))) EncodeIp<NV, TJ>::Lds lds;                  \
-    EncodeIp<NV, TJ>::run(a, lds);                                                      \
+#define EOS_TQ_ENCODE_IP(NAME, NV, TJ, P)                                               \
+  extern "C" __global__ __launch_bounds__(512) void eos_tq_encode_ip_##NAME##TJ(TqIpArgs a) { \
+    __shared__ __attribute__((aligned(16))) EncodeIp<NV, TJ, P>::Lds lds;               \
+    EncodeIp<NV, TJ, P>::run(a, lds);                                                   \
   }
-EOS_TQ_ENCODE_IP(2, 1)
-EOS_TQ_ENCODE_IP(2, 2)
-EOS_TQ_ENCODE_IP(2, 3)
-EOS_TQ_ENCODE_IP(2, 4)
-EOS_TQ_ENCODE_IP(1, 5)
-EOS_TQ_ENCODE_IP(1, 6)
-EOS_TQ_ENCODE_IP(1, 7)
-EOS_TQ_ENCODE_IP(1, 8)
+EOS_TQ_ENCODE_IP(t, 2, 1, 4)
+EOS_TQ_ENCODE_IP(t, 2, 2, 4)
+EOS_TQ_ENCODE_IP(t, 2, 3, 4)
+EOS_TQ_ENCODE_IP(t, 2, 4, 4)
+EOS_TQ_ENCODE_IP(t, 1, 5, 4)
+EOS_TQ_ENCODE_IP(t, 1, 6, 4)
+EOS_TQ_ENCODE_IP(t, 1, 7, 4)
+EOS_TQ_ENCODE_IP(t, 1, 8, 4)
+EOS_TQ_ENCODE_IP(s, 1, 1, 8)
+EOS_TQ_ENCODE_IP(s, 1, 2, 8)
+EOS_TQ_ENCODE_IP(s, 1, 3, 8)
+EOS_TQ_ENCODE_IP(s, 1, 4, 8)
+EOS_TQ_ENCODE_IP(s, 1, 5, 8)
+EOS_TQ_ENCODE_IP(s, 1, 6, 8)
+EOS_TQ_ENCODE_IP(s, 1, 7, 8)
+EOS_TQ_ENCODE_IP(s, 1, 8, 8)
 #undef EOS_TQ_ENCODE_IP

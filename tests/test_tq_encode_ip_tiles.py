@@ -1,4 +1,4 @@
-"""The inner-product encode on the f64 matrix cores (eos_tq_encode_ip_t*):
+"""The inner-product encode on the f64 matrix cores (eos_tq_encode_ip_s*, _t*):
 codes, signs, ResNorm and Norm bit-exact against the CPU oracle at the edges
 of its tiles (16 rows and vectors, 128 coordinates per kernel variant, 32 or
 16 vectors per workgroup, 64-wide K chunks), with zero, infinite and NaN
@@ -43,3 +43,22 @@ def test_encode_ip_tiles_bit_exact(rt, d, bits, n, rotate):
     for g, w in zip(got, want):
         np.testing.assert_array_equal(g, w)
     iq.release()
+
+
+@pytest.mark.parametrize("d,bits", [(24, 2), (130, 3), (300, 1), (512, 4), (520, 3), (1000, 2)])
+def test_encode_ip_large_calls_equal_small_ones(rt, d, bits):
+    """Calls above 16 vectors a CU take workgroups of 32 vectors (16 above dim
+    512) and shorter loads; the same vectors in calls of 1,111 do not."""
+    n = 16 * 256 + 37
+    print(f"[case] ip encode large d={d} bits={bits} n={n}", flush=True)
+    rng = np.random.default_rng(d + bits)
+    rot = np.linalg.qr(rng.normal(size=(d, d)))[0].astype(np.float32)
+    S = rng.normal(size=(d, d)).astype(np.float32)
+    cb = np.linspace(-127, 127, 1 << bits).round().astype(np.int8)
+    x = rng.normal(size=(n, d)).astype(np.float32)
+    x[4100] = 0
+    qz = IPQuantizer(rt, d, bits, cb, float(np.float32(2.5 / np.sqrt(d) / 127)), rot, S)
+    whole = qz.encode(x)
+    parts = [qz.encode(x[i:i + 1111]) for i in range(0, n, 1111)]
+    for w, *p in zip(whole, *parts):
+        np.testing.assert_array_equal(w, np.concatenate(p))
