@@ -1184,7 +1184,7 @@ int rank_chunks(EosHipRuntime* rt, int rows, int64_t n, int kk) {
 // a kk too large to merge) one workgroup ranks each row.
 int rank_rows(EosHipRuntime* rt, const float* d_rows, int rows, int64_t n, int kk, int64_t* d_ids,
               float* d_scores, unsigned long long* keys, uint32_t* counts, int* status,
-              const char* label, char** err) {
+              const char* label, char** err, int least_chunks = 2) {
   TqSelectArgs sel;
   memset(&sel, 0, sizeof(sel));
   sel.rows = d_rows;
@@ -1195,7 +1195,7 @@ int rank_rows(EosHipRuntime* rt, const float* d_rows, int rows, int64_t n, int k
   sel.kk = kk;
   sel.nrows = rows;
   const int nch = rank_chunks(rt, rows, n, kk);
-  if (nch <= 1) {
+  if (nch < least_chunks) {
     sel.mode = 1;
     return rt->launch("eos_tq_row_select", dim3(rows), dim3(1024), 0, &sel, err, label);
   }
@@ -1516,6 +1516,10 @@ struct EosHipTQParents {
 
 namespace {
 
+// Chunks from which a parent row's ranking is split: below 16,384 parents one
+// workgroup a row costs no more than the merge's launch.
+constexpr int kParentChunks = 8;
+
 // Queries per pass: the dense child-score block [per][n] stays under 4 GiB.
 int parent_batch(const EosHipTQParents* P) {
   const int64_t by_mem = ((int64_t)1 << 32) / std::max<int64_t>(1, P->tq->n * 4);
@@ -1579,7 +1583,8 @@ int parent_topk_impl(EosHipRuntime* rt, EosHipTQParents* P, const float* d_queri
     }
     // The flat scan's candidate lists (kBatch x kCap keys) hold the chunks'.
     if (rank_rows(rt, P->pscores, qb, P->np, kk, d_ids + (size_t)q0 * kk, d_scores + (size_t)q0 * kk,
-                  tq->cand, tq->cand_count, tq->status, "tq_parent_select", err) != 0)
+                  tq->cand, tq->cand_count, tq->status, "tq_parent_select", err,
+                  kParentChunks) != 0)
       return 1;
     TqParentBestArgs bb;
     memset(&bb, 0, sizeof(bb));
