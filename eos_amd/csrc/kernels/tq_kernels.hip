@@ -1767,23 +1767,34 @@ extern "C" __global__ __launch_bounds__(kSelThreads) void eos_tq_row_select(TqSe
       if (((c ^ pfx) & hmask) == 0ull) atomicAdd(&hist[(c >> shift) & 255u], 1u);
     });
     __syncthreads();
-    if (tid == 0) {
-      int rem = sel_rem;
-      uint32_t cum = 0;
-      int digit = 0;
-      for (int b = 255; b >= 0; --b) {
-        if (cum + hist[b] >= (uint32_t)rem) {
-          digit = b;
-          rem -= (int)cum;
-          break;
-        }
-        cum += hist[b];
+    // The digit's bin, from the top: lane l of the first wavefront sums bins
+    // 255 - 4 l .. 252 - 4 l, a prefix sum over the lanes finds the bin. (One
+    // thread's walk, an LDS read per bin, was most of the kernel: 16 rows of
+    // 40,000 in 16 chunks, k = 50, 34 -> 10 us.)
+    if (tid < 64) {
+      const uint32_t rem = (uint32_t)sel_rem;
+      uint32_t h[4], tot = 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        h[e] = hist[255 - 4 * tid - e];
+        tot += h[e];
       }
-      sel_rem = rem;
-      sel_prefix = pfx | ((u64)digit << shift);
-      // Selecting a set (modes 1, 2): once every element under the prefix
-      // is needed, the keys >= the prefix (lower digits 0) are exactly kk.
-      if (a.mode != 0 && hist[digit] == (uint32_t)rem) sel_done = 1;
+      uint32_t incl = tot;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t t = (uint32_t)__shfl_up((int)incl, o);
+        if (tid >= o) incl += t;
+      }
+      uint32_t cum = incl - tot;
+      if (cum < rem && incl >= rem) {
+        int e = 0;
+        while (cum + h[e] < rem) cum += h[e++];
+        sel_rem = (int)(rem - cum);
+        sel_prefix = pfx | ((u64)(255 - 4 * tid - e) << shift);
+        // Selecting a set (modes 1, 2): once every element under the prefix
+        // is needed, the keys >= the prefix (lower digits 0) are exactly kk.
+        if (a.mode != 0 && h[e] == rem - cum) sel_done = 1;
+      }
     }
     __syncthreads();
   }
