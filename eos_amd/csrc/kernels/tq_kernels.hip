@@ -2616,7 +2616,8 @@ EOS_TQ_MAXSIM(4, 32, 1)
 // the wave pops the best min(top_n, count) values in descending order --
 // the order aggregateMultiVectorParentScores sums the accumulator's list in
 // (runtime/retrieval_multivector_turboquant.go:769-810) -- and forms the
-// parent score in f64 with explicitly rounded operations.
+// parent score in f64 with explicitly rounded operations. A NaN child score
+// (an overflowed product times a zero Norm) counts as -infinity.
 extern "C" __global__ __launch_bounds__(256) void eos_tq_parent_agg(TqParentArgs a) {
   const int lane = threadIdx.x & 63;
   const long long i = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -2645,7 +2646,8 @@ extern "C" __global__ __launch_bounds__(256) void eos_tq_parent_agg(TqParentArgs
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (base + 64LL * u < c1) {
-        float x = v[u];
+        // (a NaN would leave the score before it in two places)
+        float x = v[u] == v[u] ? v[u] : -__builtin_inff();
 #pragma unroll
         for (int i = 0; i < 5; ++i) {
           const float hi = fmaxf(x, t[i]), lo = fminf(x, t[i]);
@@ -2708,7 +2710,8 @@ extern "C" __global__ __launch_bounds__(256) void eos_tq_parent_agg_short(TqPare
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (base + u < n) {
-        float x = v[u];
+        // (a NaN would leave the score before it in two places)
+        float x = v[u] == v[u] ? v[u] : -__builtin_inff();
 #pragma unroll
         for (int i = 0; i < 5; ++i) {
           const float hi = fmaxf(x, t[i]), lo = fminf(x, t[i]);
