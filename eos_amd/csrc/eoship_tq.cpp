@@ -412,7 +412,7 @@ struct EosHipTQ {
   }
 
   // Arguments of a MaxSim launch over the prepared chunk's groups [g0, g0 +
-  // groups) (passes of maxsim_nqg() groups on blockIdx.y).
+  // groups) (maxsim_launch splits them into passes on blockIdx.y).
   TqMaxsimArgs maxsim_args(int g0, int groups, int doc_len) const {
     TqMaxsimArgs m;
     memset(&m, 0, sizeof(m));
@@ -1260,15 +1260,16 @@ int maxsim_filtered(EosHipRuntime* rt, EosHipTQ* tq, int doc_len, int64_t ndocs,
   r = std::max(r, std::min(safe, room));
   r = std::max<int64_t>(1, std::min<int64_t>(r, ns));
   // workspace: samples [cq][ns] f32, tau [cq], lists [cq][kMsList] u32, list
-  // counts [cq] and key counts [cq] (cleared together), rank keys
-  // [cq][kMsCap] u64, status [cq]
+  // counts [cq][EOS_MS_COUNT] and key counts likewise (cleared together), rank
+  // keys [cq][kMsCap] u64, status [cq]
   auto al = [](size_t b) { return (b + 255) / 256 * 256; };
   const size_t o_samp = 0;
   const size_t o_tau = o_samp + al((size_t)cq * ns * 4);
   const size_t o_list = o_tau + al((size_t)cq * 4);
   const size_t o_lcnt = o_list + al((size_t)cq * kMsList * 4);
-  const size_t o_ccnt = o_lcnt + (size_t)cq * 4;
-  const size_t o_cand = o_lcnt + al((size_t)cq * 8);
+  const size_t count_bytes = (size_t)cq * EOS_MS_COUNT * 4;
+  const size_t o_ccnt = o_lcnt + count_bytes;
+  const size_t o_cand = o_ccnt + count_bytes;
   const size_t o_stat = o_cand + al((size_t)cq * kMsCap * 8);
   const size_t total = o_stat + al((size_t)cq * 4);
   if (tq->ensure(&tq->ms_ws, &tq->ms_ws_bytes, total, err) != 0) return 1;
@@ -1299,7 +1300,7 @@ int maxsim_filtered(EosHipRuntime* rt, EosHipTQ* tq, int doc_len, int64_t ndocs,
   if (rt->launch("eos_tq_threshold", dim3((unsigned)cq), dim3(256), 0, &sel, err, "tq_maxsim_threshold") != 0)
     return 1;
   // 2. bound filter
-  hipError_t e = hipMemsetAsync(lcnt, 0, (size_t)cq * 8, rt->stream);
+  hipError_t e = hipMemsetAsync(lcnt, 0, 2 * count_bytes, rt->stream);
   if (e != hipSuccess) return hip_err(err, "hipMemsetAsync(list counts)", e);
   m = tq->maxsim_args(0, cq, doc_len);
   m.doc_begin = 0;
@@ -1332,6 +1333,7 @@ int maxsim_filtered(EosHipRuntime* rt, EosHipTQ* tq, int doc_len, int64_t ndocs,
   f.cap = kMsCap;
   f.kk = kk;
   f.q = cq;
+  f.count_stride = EOS_MS_COUNT;
   if (rt->launch(finalize_kernel(f.kk), dim3((unsigned)cq), dim3(256), 0, &f, err, "tq_maxsim_finalize") != 0)
     return 1;
   // 4. exhaustive rows of the flagged queries (both launches return at once

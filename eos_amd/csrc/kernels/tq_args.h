@@ -86,6 +86,7 @@ struct TqFinalizeArgs {
   float* scores;      // [q][kk]
   int* status;        // [q]: 0 ok, 1 too few candidates, 2 overflow
   int cap, kk, q;
+  int count_stride;       // of cand_count, in counters (0 = 1)
   const long long* id_map;  // optional [n]: corpus position p is reported as id id_map[p]
 };
 
@@ -110,11 +111,12 @@ struct TqMaxsimArgs {
   // Pass p = blockIdx.y scores query groups [nqg p, nqg p + nqg) of the
   // launch (alpha, out, tau, gate, lonorm and the doc lists offset by it).
   // Document i of a pass is doc_begin + i * doc_stride (doc_stride 0 = 1),
-  // or, with doc_list, doc_list[p * list_cap + i] for i < min(count, cap),
-  // count = list_count[p]; in that mode the exact scores >= tau[group] are
-  // appended as rank keys to cand[group * cand_cap ..], counted in
-  // cand_count[group] (cleared by the caller; entries past cand_cap dropped),
-  // which an overflowed list raises by 2^30.
+  // or, with doc_list (kernels of one group a pass only), doc_list[group *
+  // list_cap + i] for i < min(count, cap), count = list_count[group]; in that
+  // mode the exact scores >= tau[group] are appended as rank keys to
+  // cand[group * cand_cap ..], counted in cand_count[group] (cleared by the
+  // caller; entries past cand_cap dropped), which an overflowed list raises by
+  // 2^30.
   long long doc_stride;
   const uint32_t* doc_list;
   unsigned long long* cand;
@@ -130,13 +132,18 @@ struct TqMaxsimArgs {
   uint32_t* list_count;
   int list_cap, cand_cap;
 };
+// Counters of a group lie this many uint32 apart (list_count and cand_count
+// above are [group * EOS_MS_COUNT]): 256 bytes, so that the groups' atomics do
+// not queue for one cache line.
+#define EOS_MS_COUNT 64
+
+// Children up to which one lane aggregates a parent (eos_tq_parent_agg_short).
+#define EOS_PARENT_SHORT 64
 
 // Parent (multivector) aggregation over child scores: parent p owns children
 // [off[p], off[p+1]) of each score row; out[q][p] = f32(mean of its best
 // min(top_n, 5, count) child scores (f64 sum in descending order) -
 // penalty * l1p[p]); parents without children get -inf.
-// Children up to which one lane aggregates a parent (eos_tq_parent_agg_short).
-#define EOS_PARENT_SHORT 64
 struct TqParentArgs {
   const float* scores;      // [qb][stride] child scores
   const long long* off;     // [np + 1]
