@@ -1242,6 +1242,18 @@ constexpr int kMsTarget = 1024;
 constexpr int kMsSampleDocs = 2048;
 constexpr int kMsMinDocs = 16384;
 constexpr int kMsMaxK = 512;
+// Least r with P(N >= r) <= 1 / 3000 for a Poisson count N of this mean.
+int64_t maxsim_safe_rank(double mean) {
+  double p = std::exp(-mean), below = p;  // P(N = r - 1), P(N < r)
+  int64_t r = 1;
+  while (1.0 - below > 1.0 / 3000 && r < kMsSampleDocs) {
+    p *= mean / (double)r;
+    below += p;
+    ++r;
+  }
+  return r;
+}
+
 int maxsim_filtered(EosHipRuntime* rt, EosHipTQ* tq, int doc_len, int64_t ndocs, int cq, int kk,
                     int64_t* d_ids, float* d_scores, char** err) {
   const int64_t stride = std::max<int64_t>(16, (ndocs + kMsSampleDocs - 1) / kMsSampleDocs);
@@ -1249,13 +1261,13 @@ int maxsim_filtered(EosHipRuntime* rt, EosHipTQ* tq, int doc_len, int64_t ndocs,
   const double target = std::min<double>(3.0 * kk, kMsTarget);
   int64_t r = (int64_t)std::ceil(target * (double)ns / (double)ndocs);
   // Fewer than kk documents score >= tau when r or more of the sample are
-  // among the best kk, a Poisson count of mean x: r of at least x + 3 sqrt(x)
-  // + 2 makes that about one query in 3,000 (at 100,000 documents and k = 100
-  // 3 kk alone, r = 7, one in 200: with 32 queries every seventh call paid an
-  // exhaustive pass, 1.5 ms, where two more list entries in seven cost 40
-  // us), unless so many documents above tau would crowd the kept keys.
-  const double x = (double)kk * (double)ns / (double)ndocs;
-  const int64_t safe = (int64_t)std::ceil(x + 3.0 * std::sqrt(x) + 2.0);
+  // among the best kk - 1, a Poisson count of mean (kk - 1) ns / ndocs: r is
+  // raised until that is one query in 3,000 or rarer (at 100,000 documents and
+  // k = 100 3 kk alone, r = 7, gives one in 200: with 32 queries every seventh
+  // call paid an exhaustive pass, 1.5 ms, where two more list entries in seven
+  // cost 40 us), unless so many documents above tau would crowd the kept keys.
+  // The best of the sample (r = 1) always does for kk = 1.
+  const int64_t safe = maxsim_safe_rank((double)(kk - 1) * (double)ns / (double)ndocs);
   const int64_t room = (int64_t)((double)(kMsCap / 2) * (double)ns / (double)ndocs);
   r = std::max(r, std::min(safe, room));
   r = std::max<int64_t>(1, std::min<int64_t>(r, ns));
