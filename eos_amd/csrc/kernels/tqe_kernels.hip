@@ -76,9 +76,13 @@ constexpr int kSplitStage = 4;     // staging wavefronts
 // two sides and whether it is a decision point. Values closer to one than
 // delta2 = 2 E / s_c (+ 1e-4 for the rounding of w) go to a list and are
 // decided in f64: first from a sum in another order with its own bound, then,
-// if that is not enough (exact ties), by the contract's fma chain. The list
-// holds about 1 of 600 coordinates at d = 384, 4 bits; when it overflows every
-// pair of the workgroup is decided that way.
+// if that is not enough (exact ties), by the contract's fma chain, a thread
+// each. The list holds about 1 of 600 coordinates at d = 384, 4 bits. When it
+// overflows (sparse vectors under a rotation of few nonzeros: every zero is a
+// tie of a symmetric codebook) the tile is decided on the f64 matrix cores:
+// 20,000 x 384 under a signed permutation, half of the values zero, 218 us
+// (f64 VALU chains for every vector 678; each pair by 16 lanes and then one
+// 22,748), a hundredth of them zero, a list of ties, 107 (686; 434).
 // The norm's f64 sum is taken in another order too: it is kept when the f32
 // norms of its two error bounds agree, else recomputed as the chain.
 // A vector of norm 0 has u = 0 and every distance 0, one of infinite or NaN
@@ -113,7 +117,7 @@ struct EncodeSplit {
     double s64[BM];
     float inv2[BM], dlim[BM];
     uint32_t items[kSplitItems];
-    uint32_t nitems;
+    uint32_t nitems, nties;
     uint16_t lut[512];
   };
   const TqEncSplitArgs& a;
@@ -166,7 +170,7 @@ struct EncodeSplit {
       }
       s.lut[i] = (uint16_t)(a.li[below] | (a.li[upto] << 4) | (upto != below ? 0x1000 : 0));
     }
-    if (wave == 0 && lane == 0) s.nitems = 0u;
+    if (wave == 0 && lane == 0) s.nitems = s.nties = 0u;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) tot[rt] = v16f{0};
     lds_barrier();
@@ -229,12 +233,39 @@ struct EncodeSplit {
     }
   }
 
-  // Pair i of the list (or of the whole tile) by 16 lanes: every lane's
-  // 16-byte pieces of the two rows are requested six at a time.
-  EOS_DEV void decide(int i, bool all, int jn, int sub) {
+  EOS_DEV void put_code(int v, int jl, int code) {
+    const int bit = jl * a.bits;
+    const int off = v * CST + (bit >> 3), sh = (off & 3) * 8 + (bit & 7);
+    uint32_t* word = reinterpret_cast<uint32_t*>(&s.cbuf[off & ~3]);
+    atomicAnd(word, ~(((1u << a.bits) - 1u) << sh));
+    atomicOr(word, (uint32_t)code << sh);
+  }
+
+  // The contract's decisions for N values u of a vector of norm ne.
+  template <int N>
+  EOS_DEV void nearest(const double (&u)[N], double ne, int (&code)[N]) {
+    double bd[N];
+#pragma unroll 1
+    for (int l = 0; l < (1 << a.bits); ++l) {
+      const double nc = ne * ((double)a.cb_scale * (double)a.cb[l]);
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const double dv = fabs(u[i] - nc);
+        if (l == 0 || dv < bd[i]) {
+          bd[i] = dv;
+          code[i] = l;
+        }
+      }
+    }
+  }
+
+  // Pair i of the list by 16 lanes: every lane's 16-byte pieces of the two
+  // rows are requested six at a time. Pairs that this leaves open go to the
+  // ties (in xs, which nothing reads any more).
+  EOS_DEV void decide(int i, int sub) {
     const int d = a.d;
-    const int v = all ? i / jn : (int)(s.items[i] >> 16);
-    const int jl = all ? i - v * jn : (int)(s.items[i] & 0xffffu);
+    const uint32_t item = s.items[i];
+    const int v = (int)(item >> 16), jl = (int)(item & 0xffffu);
     if (s.dlim[v] < -1.0f) return;
     const float* xv = a.x + (size_t)(v0 + v) * d;
     const float* rj = a.rot_r + (size_t)(32 * jt0 + jl) * d;
@@ -290,31 +321,150 @@ struct EncodeSplit {
     }
     const double err = (4.0 * d + 32.0) * 2.220446049250313e-16 * nrm *
                        ((double)a.rmax + 128.0 * (double)a.cb_scale);
-    if (!(d2 - d1 > 2.0 * err)) {
-      // The contract's own chain.
-      double ue = 0.0, se = 0.0;
+    if (d2 - d1 > 2.0 * err)
+      put_code(v, jl, code);
+    else
+      (&s.xs[0][0][0])[atomicAdd(&s.nties, 1u)] = item;
+  }
+
+  // A tie by the contract's own chains, one thread each: 16 values of either
+  // row are requested at a time.
+  EOS_DEV void tie(uint32_t item) {
+    const int d = a.d, v = (int)(item >> 16), jl = (int)(item & 0xffffu);
+    const float* xv = a.x + (size_t)(v0 + v) * d;
+    const float* rj = a.rot_r + (size_t)(32 * jt0 + jl) * d;
+    double u[1] = {0.0}, ss = 0.0;
 #pragma unroll 1
-      for (int k = 0; k < d; ++k) {
-        ue = fma((double)rj[k], (double)xv[k], ue);
-        se = fma((double)xv[k], (double)xv[k], se);
+    for (int k0 = 0; k0 < d; k0 += 16) {
+      float xk[16], rk[16];
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        load4(xk + 4 * p, xv, k0 + 4 * p);
+        load4(rk + 4 * p, rj, k0 + 4 * p);
       }
-      const double ne = __builtin_sqrt(se);
-      double bd = 0.0;
-      code = 0;
-#pragma unroll 1
-      for (int l = 0; l < (1 << a.bits); ++l) {
-        const double dv = fabs(ue - ne * ((double)a.cb_scale * (double)a.cb[l]));
-        if (l == 0 || dv < bd) {
-          bd = dv;
-          code = l;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        if (k0 + e < d) {
+          u[0] = fma((double)rk[e], (double)xk[e], u[0]);
+          ss = fma((double)xk[e], (double)xk[e], ss);
         }
       }
     }
-    const int bit = jl * a.bits;
-    const int off = v * CST + (bit >> 3), sh = (off & 3) * 8 + (bit & 7);
-    uint32_t* word = reinterpret_cast<uint32_t*>(&s.cbuf[off & ~3]);
-    atomicAnd(word, ~(((1u << a.bits) - 1u) << sh));
-    atomicOr(word, (uint32_t)code << sh);
+    int code[1];
+    nearest(u, __builtin_sqrt(ss), code);
+    put_code(v, jl, code[0]);
+  }
+
+  // Values k .. k + 3 of a row (positions clamped to its end).
+  EOS_DEV void load4(float* out, const float* row, int k) {
+    if constexpr (VEC) {
+      const float4 f = *reinterpret_cast<const float4*>(row + min(k, a.d - 4));
+      out[0] = f.x;
+      out[1] = f.y;
+      out[2] = f.z;
+      out[3] = f.w;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) out[e] = row[min(k + e, a.d - 1)];
+    }
+  }
+  // The operands of four v_mfma_f64_16x16x4_f64 steps, K values k0 .. k0 + 15
+  // (zero past d) of the lane's row: lane group g loads values 4 g .. + 3 and
+  // needs value g of each step, a 4 x 4 transposition across the groups.
+  EOS_DEV void load_steps(float (&f)[4], const float* row, int k0, int g) {
+    load4(f, row, k0 + 4 * g);
+    uint32_t u[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) u[e] = k0 + 4 * g + e < a.d ? __float_as_uint(f[e]) : 0u;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const auto r = __builtin_amdgcn_permlane32_swap(u[e], u[e + 2], false, false);
+      u[e] = r[0];
+      u[e + 2] = r[1];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e += 2) {
+      const auto r = __builtin_amdgcn_permlane16_swap(u[e], u[e + 1], false, false);
+      u[e] = r[0];
+      u[e + 1] = r[1];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) f[e] = __uint_as_float(u[e]);
+  }
+
+  // Every pair of the tile by the contract, for a list that overflowed: u on
+  // v_mfma_f64_16x16x4_f64, whose chain over K is the contract's fma chain
+  // (see EncodeIp), 3 x 3 tiles of 16 coordinates x 16 vectors a wavefront;
+  // the vectors' norms by a thread each. Bound by the f64 matrix rate.
+  EOS_DEV void exact_tile(int tid) {
+    const int d = a.d, lane = tid & 63, lr = lane & 15, g = lane >> 4;
+    for (int v = tid; v < nv; v += NT) {
+      const float* xv = a.x + (size_t)(v0 + v) * d;
+      double ss = 0.0;
+#pragma unroll 1
+      for (int k0 = 0; k0 < d; k0 += 16) {
+        float xk[16];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) load4(xk + 4 * p, xv, k0 + 4 * p);
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if (k0 + e < d) ss = fma((double)xk[e], (double)xk[e], ss);
+      }
+      s.s64[v] = __builtin_sqrt(ss);
+    }
+    lds_barrier();
+    const int jn = min(32 * NW, d - 32 * jt0);
+    const int jg = (jn + 47) / 48, vg = (nv + 47) / 48;
+#pragma unroll 1
+    for (int it = tid >> 6; it < jg * vg; it += NT / 64) {
+      const int jb = it % jg * 48 + lr, vb = it / jg * 48 + lr;
+      const float *rj[3], *xv[3];
+#pragma unroll
+      for (int t = 0; t < 3; ++t) {
+        rj[t] = a.rot_r + (size_t)(32 * jt0 + min(jb + 16 * t, jn - 1)) * d;
+        xv[t] = a.x + (size_t)(v0 + min(vb + 16 * t, nv - 1)) * d;
+      }
+      v4d acc[3][3];
+#pragma unroll
+      for (int n = 0; n < 3; ++n)
+#pragma unroll
+        for (int t = 0; t < 3; ++t) acc[n][t] = v4d{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
+      for (int k0 = 0; k0 < d; k0 += 16) {
+        float rf[3][4], xf[3][4];
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+          load_steps(rf[t], rj[t], k0, g);
+          load_steps(xf[t], xv[t], k0, g);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int n = 0; n < 3; ++n)
+#pragma unroll
+            for (int t = 0; t < 3; ++t)
+              acc[n][t] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)rf[t][e], (double)xf[n][e],
+                                                               acc[n][t], 0, 0, 0);
+      }
+      // Element r of a lane: coordinate jb - lr + g + 4 r, vector vb.
+#pragma unroll
+      for (int n = 0; n < 3; ++n) {
+        const int v = vb + 16 * n;
+        if (v >= nv) continue;
+        const double ne = s.s64[v];
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+          const double u[4] = {acc[n][t][0], acc[n][t][1], acc[n][t][2], acc[n][t][3]};
+          int code[4];
+          nearest(u, ne, code);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int jl = jb - lr + 16 * t + g + 4 * r;
+            if (jl < jn) put_code(v, jl, code[r]);
+          }
+        }
+      }
+    }
   }
 
   // Code rows: the tile's bytes of each vector.
@@ -455,11 +605,16 @@ struct EncodeSplit {
     else
       stage(tid - 64 * NW);
     lds_barrier();
-    const bool all = s.nitems > (uint32_t)kSplitItems;
-    const int jn = min(32 * NW, a.d - 32 * jt0);
-    const int total = all ? nv * jn : (int)s.nitems;
+    if (s.nitems > (uint32_t)kSplitItems) {
+      exact_tile(tid);
+    } else {
+      const int total = (int)s.nitems;
 #pragma unroll 1
-    for (int i = tid >> 4; i < total; i += NT / 16) decide(i, all, jn, tid & 15);
+      for (int i = tid >> 4; i < total; i += NT / 16) decide(i, tid & 15);
+      lds_barrier();
+      const uint32_t* ties = &s.xs[0][0][0];
+      for (int i = tid; i < (int)s.nties; i += NT) tie(ties[i]);
+    }
     lds_barrier();
     write(tid);
   }

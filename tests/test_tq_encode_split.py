@@ -65,3 +65,25 @@ def test_encode_split_undecided_vectors(rt, d):
     with np.errstate(all="ignore"):
         _check(rt, x, rot, d, 4)
         _check(rt, x[58:70], datagen.orthogonal(d + 9, d).astype(np.float32), d, 2)
+
+
+@pytest.mark.parametrize("d,bits", [(1, 4), (16, 4), (33, 2), (47, 4), (100, 2), (130, 4), (384, 4),
+                                    (385, 4), (770, 2), (1024, 4)])
+def test_encode_split_ties(rt, d, bits):
+    """Zeros under a signed permutation are exact ties of the symmetric
+    levels: few of them (a thread's chains each), too many for a tile's list
+    (the whole tile on f64 MFMA), and a tile of tiny vectors, which leave
+    every coordinate to the list."""
+    print(f"[case] split encode ties d={d} bits={bits}", flush=True)
+    rng = np.random.default_rng(d)
+    rot = np.zeros((d, d), np.float32)
+    rot[np.arange(d), rng.permutation(d)] = np.where(np.arange(d) % 2 == 0, 1.0, -1.0)
+    x = rng.normal(size=(3 * 96 + 50, d)).astype(np.float32)
+    x[:96][rng.random((96, d)) < 0.01] = 0
+    x[96:192][rng.random((96, d)) < 0.6] = 0
+    x[192:288] *= np.float32(1e-31)
+    x[288:, : (d + 1) // 2] = 0
+    with np.errstate(all="ignore"):
+        x[200, 0], x[201, d - 1], x[202] = np.inf, np.nan, 0
+        _check(rt, x, rot, d, bits)
+        _check(rt, x[192:230], datagen.orthogonal(d + 9, d).astype(np.float32), d, bits)
