@@ -2697,7 +2697,7 @@ extern "C" __global__ __launch_bounds__(256) void eos_tq_parent_agg(TqParentArgs
     for (int u = 0; u < U; ++u) {
       if (base + 64LL * u < c1) {
         // (a NaN would leave the score before it in two places)
-        float x = v[u] == v[u] ? v[u] : -__builtin_inff();
+        float x = fmaxf(v[u], -__builtin_inff());
 #pragma unroll
         for (int i = 0; i < 5; ++i) {
           const float hi = fmaxf(x, t[i]), lo = fminf(x, t[i]);
@@ -2761,7 +2761,7 @@ extern "C" __global__ __launch_bounds__(256) void eos_tq_parent_agg_short(TqPare
     for (int u = 0; u < U; ++u) {
       if (base + u < n) {
         // (a NaN would leave the score before it in two places)
-        float x = v[u] == v[u] ? v[u] : -__builtin_inff();
+        float x = fmaxf(v[u], -__builtin_inff());
 #pragma unroll
         for (int i = 0; i < 5; ++i) {
           const float hi = fmaxf(x, t[i]), lo = fminf(x, t[i]);
