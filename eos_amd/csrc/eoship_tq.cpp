@@ -1184,7 +1184,7 @@ int rank_chunks(EosHipRuntime* rt, int rows, int64_t n, int kk) {
 // a kk too large to merge) one workgroup ranks each row.
 int rank_rows(EosHipRuntime* rt, const float* d_rows, int rows, int64_t n, int kk, int64_t* d_ids,
               float* d_scores, unsigned long long* keys, uint32_t* counts, int* status,
-              const char* label, char** err, int least_chunks = 2) {
+              const char* label, char** err, bool split = true) {
   TqSelectArgs sel;
   memset(&sel, 0, sizeof(sel));
   sel.rows = d_rows;
@@ -1194,8 +1194,8 @@ int rank_rows(EosHipRuntime* rt, const float* d_rows, int rows, int64_t n, int k
   sel.stride = n;
   sel.kk = kk;
   sel.nrows = rows;
-  const int nch = rank_chunks(rt, rows, n, kk);
-  if (nch < least_chunks) {
+  const int nch = split ? rank_chunks(rt, rows, n, kk) : 1;
+  if (nch < 2) {
     sel.mode = 1;
     return rt->launch("eos_tq_row_select", dim3(rows), dim3(1024), 0, &sel, err, label);
   }
@@ -1530,9 +1530,15 @@ struct EosHipTQParents {
 
 namespace {
 
-// Chunks from which a parent row's ranking is split: below 16,384 parents one
-// workgroup a row costs no more than the merge's launch.
-constexpr int kParentChunks = 8;
+// Whether a parent row's ranking is split. The merge of the chunks' best costs
+// a launch and, at large k, a sort of k keys; one workgroup a row costs about
+// 1 us per 1,000 parents. Whole calls, split against one workgroup a row:
+// 8,320 parents, k = 50, 2 queries 36 / 36 us; 16,384 37 / 42, 64 queries
+// 58 / 63; 40,000, 16 queries, k = 100 54 / 76, k = 1,000 131 / 99; 64 queries,
+// k = 100 87 / 111. The second line passes through the sizes at which both cost
+// the same: 16,000 parents at k = 300, 24,000 at 400, 41,000 at 600, 60,000 at
+// 800, 76,000 at 1,000.
+bool parents_split(int64_t np, int kk) { return np >= 16384 && np >= 84 * (int64_t)kk - 9600; }
 
 // Queries per pass: the dense child-score block [per][n] stays under 4 GiB.
 int parent_batch(const EosHipTQParents* P) {
@@ -1598,7 +1604,7 @@ int parent_topk_impl(EosHipRuntime* rt, EosHipTQParents* P, const float* d_queri
     // The flat scan's candidate lists (kBatch x kCap keys) hold the chunks'.
     if (rank_rows(rt, P->pscores, qb, P->np, kk, d_ids + (size_t)q0 * kk, d_scores + (size_t)q0 * kk,
                   tq->cand, tq->cand_count, tq->status, "tq_parent_select", err,
-                  kParentChunks) != 0)
+                  parents_split(P->np, kk)) != 0)
       return 1;
     TqParentBestArgs bb;
     memset(&bb, 0, sizeof(bb));

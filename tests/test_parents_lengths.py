@@ -45,3 +45,33 @@ def test_parent_lengths_match_oracle(rt, name, counts, k):
     np.testing.assert_array_equal(sc, ws)
     par.release()
     idx.release()
+
+
+@pytest.mark.parametrize("name,np_,nq,k", [
+    ("split, eight lists of 1024 keys, the merge's limit", 77000, 2, 1024),
+    ("split, seven lists above the smaller merge's limit", 76800, 2, 1025),
+    ("split at 64 queries", 16500, 64, 40),
+    ("just above the line", 24000, 3, 400),
+    ("just below the line", 23999, 3, 400),
+    ("large k on one workgroup a row", 33000, 2, 1000),
+])
+def test_parent_ranking_split(rt, name, np_, nq, k):
+    """Parents' ranking split into chunks and not, at the edges of the merge."""
+    from eos_amd.turboquant import TurboQuantIndex, TurboQuantParents
+    print(f"[case] parent ranking: {name}", flush=True)
+    off = np.arange(np_ + 1, dtype=np.int64)
+    c = datagen.TurboQuantCorpus(np_, 24, 2, 15, 16, 17)
+    norms = c.norms.copy()
+    norms[np_ // 2:np_ // 2 + 40] = norms[0]  # more equal scores
+    codes = c.codes.copy()
+    codes[np_ // 2:np_ // 2 + 40] = codes[0]
+    q = datagen.baseline_queries(nq, 24, 18)
+    idx = TurboQuantIndex(rt, codes, norms, 24, 2, c.codebook, c.codebook_scale, c.rotation)
+    par = TurboQuantParents(idx, off)
+    got = par.top_k(q, k, "max", 0.0)
+    want = oracle.tq_parent_topk(q, c.rotation, 24, 2, c.codebook, c.codebook_scale, codes, norms,
+                                 off, k, 1, 0.0)
+    for g, w in zip(got, want):
+        np.testing.assert_array_equal(g, w)
+    par.release()
+    idx.release()
