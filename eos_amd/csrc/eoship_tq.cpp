@@ -128,9 +128,10 @@ struct EosHipTQ {
   void* packed = nullptr;
   float* norms = nullptr;
   float* rot_t = nullptr;
-  // Encoding: R row-major and its split operand fragments (rot_frag NULL: no
-  // rotation, or scales outside the split product's bound), the largest row
-  // norm of R and the decision distance in half level steps.
+  // Encoding: the split operand fragments of R and, in the same allocation, R
+  // row-major (rot_frag NULL: no rotation, or scales outside the split
+  // product's bound), the largest row norm of R and the decision distance in
+  // half level steps.
   float* rot_r = nullptr;
   void* rot_frag = nullptr;
   float rot_rmax = 0.f, enc_delta2 = 0.f;
@@ -185,7 +186,7 @@ struct EosHipTQ {
   // reported in its place. Empty / nullptr for index order.
   long long* id_map = nullptr;
   std::vector<int64_t> rank_host;
-  // Handles sharing the corpus arrays (packed, norms, rot_t, rot_r, rot_frag,
+  // Handles sharing the corpus arrays (packed, norms, rot_t, rot_frag,
   // tile_cn, codes_rm, id_map) through eoship_tq_share; nullptr while this is the only one.
   int* corpus_refs = nullptr;
 
@@ -198,7 +199,7 @@ struct EosHipTQ {
     if (corpus_refs != nullptr && --*corpus_refs > 0) return;
     delete corpus_refs;
     corpus_refs = nullptr;
-    void* corpus[] = {packed, norms, rot_t, rot_r, rot_frag, tile_cn, codes_rm, id_map};
+    void* corpus[] = {packed, norms, rot_t, rot_frag, tile_cn, codes_rm, id_map};
     for (void* p : corpus)
       if (p) hipFree(p);
   }
@@ -238,48 +239,51 @@ struct EosHipTQ {
   // with 5 % on top for the second-order terms (d = 384: 1.1e-5). Scales that
   // would put the distance over a quarter of a half step, or leave f32 and
   // bf16 no room, keep the f64 kernels (rot_frag stays NULL).
-  int prepare_encode(const float* rot, char** err) {
-    auto bf16 = [](float v) {  // round to nearest even
-      uint32_t u;
-      memcpy(&u, &v, 4);
-      u = (u + 0x7fffu + ((u >> 16) & 1u)) & 0xffff0000u;
-      memcpy(&v, &u, 4);
-      return v;
-    };
+  // R is uploaded once; its transpose and the sums come from the device. Two
+  // uploads and passes over d^2 values on the host were most of binding a small
+  // corpus (no vectors: d = 384 1.06 ms, d = 1024 7.1, now 0.12 and 0.24).
+  int prepare_rotation(const float* rot, char** err) {
+    const size_t bytes = (size_t)d * d * sizeof(float);
+    const size_t frag_bytes = (size_t)enc_tiles() * enc_chunks() * 4096;
+    if (rt->alloc(bytes, reinterpret_cast<void**>(&rot_t), err) != 0 ||
+        rt->alloc(frag_bytes + bytes, &rot_frag, err) != 0)
+      return 1;
+    rot_r = reinterpret_cast<float*>(static_cast<char*>(rot_frag) + frag_bytes);
+    hipError_t e = rt->copy_async(rot_r, rot, bytes, hipMemcpyHostToDevice);
+    if (e != hipSuccess) return hip_err(err, "hipMemcpyAsync(rotation)", e);
+    static_assert(kMaxCols >= 3, "qrot holds the sums");
+    TqRotFragArgs f{rot_r, rot_frag, rot_t, qrot, d, enc_tiles(), enc_chunks()};
+    const unsigned threads = (unsigned)(f.jtiles * f.nchunk) * 128u;
+    std::vector<double> sums(3 * (size_t)d);
+    if (rt->launch("eos_tq_rot_transpose", dim3((unsigned)(d * d + 255) / 256), dim3(256), 0, &f,
+                   err) != 0 ||
+        rt->launch("eos_tq_rot_frag", dim3((threads + 255) / 256), dim3(256), 0, &f, err) != 0 ||
+        rt->launch("eos_tq_rot_rows", dim3((unsigned)(d + 3) / 4), dim3(256), 0, &f, err) != 0)
+      return 1;
+    e = rt->copy_async(sums.data(), qrot, sums.size() * sizeof(double), hipMemcpyDeviceToHost);
+    if (e != hipSuccess) return hip_err(err, "hipMemcpyAsync(rotation sums)", e);
+    if (rt->sync(err) != 0) return 1;
     double rmax = 0.0, lmax = 0.0, emax = 0.0;
     bool finite = true;
     for (int j = 0; j < d; ++j) {
-      double ss = 0.0, sl = 0.0, se = 0.0;
-      for (int k = 0; k < d; ++k) {
-        const float v = rot[(size_t)j * d + k];
-        const float rest = v - bf16(v), low = bf16(rest), left = rest - low;
-        ss += (double)v * v;
-        sl += (double)low * low;
-        se += (double)left * left;
-      }
-      finite = finite && std::isfinite(ss);
-      rmax = std::max(rmax, ss);
-      lmax = std::max(lmax, sl);
-      emax = std::max(emax, se);
+      finite = finite && std::isfinite(sums[j]);
+      rmax = std::max(rmax, sums[j]);
+      lmax = std::max(lmax, sums[d + j]);
+      emax = std::max(emax, sums[2 * d + j]);
     }
     rmax = std::sqrt(rmax) * (1.0 + 1e-6);
     const double bound = 1.05 * (rmax * (0x1p-18 + 33 * 0x1p-23 + enc_chunks() * 0x1p-24) +
                                  std::sqrt(emax) + std::sqrt(lmax) * 0x1p-9);
     const double delta2 = 2.0 * bound / (double)cb_scale + 1e-4;
-    if (!finite || !(rmax >= 0x1p-20 && rmax <= 0x1p20) || !(cb_scale <= 0x1p20f) || !(delta2 < 0.25))
+    if (finite && rmax >= 0x1p-20 && rmax <= 0x1p20 && cb_scale <= 0x1p20f && delta2 < 0.25) {
+      rot_rmax = (float)(rmax * (1.0 + 1e-6));
+      enc_delta2 = (float)(delta2 * (1.0 + 1e-6));
       return 0;
-    rot_rmax = (float)(rmax * (1.0 + 1e-6));
-    enc_delta2 = (float)(delta2 * (1.0 + 1e-6));
-    const size_t bytes = (size_t)d * d * sizeof(float);
-    if (rt->alloc(bytes, reinterpret_cast<void**>(&rot_r), err) != 0) return 1;
-    hipError_t e = rt->copy_sync(rot_r, rot, bytes, hipMemcpyHostToDevice);
-    if (e != hipSuccess) return hip_err(err, "hipMemcpy(rotation rows)", e);
-    if (rt->alloc((size_t)enc_tiles() * enc_chunks() * 4096, &rot_frag, err) != 0) return 1;
-    TqRotFragArgs f{rot_r, rot_frag, d, enc_tiles(), enc_chunks()};
-    const unsigned threads = (unsigned)(f.jtiles * f.nchunk) * 128u;
-    if (rt->launch("eos_tq_rot_frag", dim3((threads + 255) / 256), dim3(256), 0, &f, err) != 0)
-      return 1;
-    return rt->sync(err);
+    }
+    hipFree(rot_frag);
+    rot_r = nullptr;
+    rot_frag = nullptr;
+    return 0;
   }
 
   int ensure(void** p, size_t* have, size_t need, char** err) {
@@ -853,19 +857,8 @@ int eoship_tq_bind_corpus_opts(EosHipRuntime* rt, const EosHipTQDesc* desc, cons
       }
     }
   }
-  if (desc->rotation != nullptr) {
-    std::vector<float> rt_host((size_t)tq->d * tq->d);
-    for (int j = 0; j < tq->d; ++j)
-      for (int k = 0; k < tq->d; ++k) rt_host[(size_t)k * tq->d + j] = desc->rotation[(size_t)j * tq->d + k];
-    if (rt->alloc(rt_host.size() * sizeof(float), reinterpret_cast<void**>(&tq->rot_t), err) != 0)
-      return fail();
-    e = rt->copy_sync(tq->rot_t, rt_host.data(), rt_host.size() * sizeof(float), hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-      hip_err(err, "hipMemcpy(rotation)", e);
-      return fail();
-    }
-    if (tq->prepare_encode(desc->rotation, err) != 0) return fail();
-  }
+  if (tq->alloc_scratch(err) != 0) return fail();
+  if (desc->rotation != nullptr && tq->prepare_rotation(desc->rotation, err) != 0) return fail();
   if (!map_host.empty()) {
     if (rt->alloc(map_host.size() * sizeof(long long), reinterpret_cast<void**>(&tq->id_map), err) != 0)
       return fail();
@@ -875,7 +868,6 @@ int eoship_tq_bind_corpus_opts(EosHipRuntime* rt, const EosHipTQDesc* desc, cons
       return fail();
     }
   }
-  if (tq->alloc_scratch(err) != 0) return fail();
   *out = tq;
   return 0;
 }

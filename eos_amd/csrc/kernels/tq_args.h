@@ -210,10 +210,14 @@ struct TqEncodeArgs {
   int cb[16];
 };
 
-// Rotation as the split product's operand fragments (eos_tq_rot_frag).
+// Rotation as the split product's operand fragments (eos_tq_rot_frag), its
+// rows' sums of squares (eos_tq_rot_rows) and its transpose
+// (eos_tq_rot_transpose).
 struct TqRotFragArgs {
   const float* rot_r;      // [d][d] R, row-major
   void* frag;              // [jtiles][nchunk][2][2][64][16 bytes]
+  float* rot_t;            // [d][d] R^T
+  double* sums;            // [3][d]
   int d, jtiles, nchunk;   // 32-coordinate tiles; 32-wide K chunks (even)
 };
 

@@ -57,6 +57,35 @@ extern "C" __global__ __launch_bounds__(256) void eos_tq_rot_frag(TqRotFragArgs 
   out[64] = lv;
 }
 
+// R^T, the layout of the f64 chains and of query preparation.
+extern "C" __global__ __launch_bounds__(256) void eos_tq_rot_transpose(TqRotFragArgs a) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < a.d * a.d) a.rot_t[i] = a.rot_r[(size_t)(i % a.d) * a.d + i / a.d];
+}
+
+// Squared norms of R's rows and of what the split leaves of them, for its error
+// bound: out[0..2][j] = sum over k of R^2, of low^2 and of (R - high - low)^2.
+// One wavefront per row.
+extern "C" __global__ __launch_bounds__(256) void eos_tq_rot_rows(TqRotFragArgs a) {
+  const int lane = threadIdx.x & 63, j = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (j >= a.d) return;
+  double t[3] = {0.0, 0.0, 0.0};
+  for (int k = lane; k < a.d; k += 64) {
+    const float v = a.rot_r[(size_t)j * a.d + k];
+    const float rest = v - bf16_val(bf16_bits(v));
+    const float low = bf16_val(bf16_bits(rest)), left = rest - low;
+    t[0] = fma((double)v, (double)v, t[0]);
+    t[1] = fma((double)low, (double)low, t[1]);
+    t[2] = fma((double)left, (double)left, t[2]);
+  }
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) t[i] += __shfl_xor(t[i], o);
+    if (lane == 0) a.sums[(size_t)i * a.d + j] = t[i];
+  }
+}
+
 namespace {
 
 constexpr int kSplitRows = 96;     // vectors per workgroup
@@ -68,7 +97,7 @@ constexpr int kSplitStage = 4;     // staging wavefronts
 // f32 value becomes a bf16 pair high + low, and
 //   u~ = sum over chunks of (Rh xl + Rl xh + Rh xh)
 // on bf16 MFMA, every chunk into a fresh accumulator that is then added in
-// f32. The host's bound E on |u~ - u| / |x| (prepare_encode) covers the split,
+// f32. The host's bound E on |u~ - u| / |x| (prepare_rotation) covers the split,
 // the 32 large products of a chunk summed in f32 in any order and the sum over
 // the chunks. In half steps of the integer level grid, w = 2 u~ / (nrm s_c),
 // the decision points are whole numbers (sums of neighbouring levels): a
