@@ -23,15 +23,25 @@ using eoship::set_err;
 namespace {
 
 // IEEE binary16 bits of an int8 code (every value in [-128, 127] is exact).
-uint16_t int8_to_f16_bits(int8_t x) {
+constexpr uint16_t f16_bits(int x) {
   if (x == 0) return 0;
   const uint16_t sign = x < 0 ? 0x8000 : 0;
-  unsigned v = (unsigned)(x < 0 ? -(int)x : (int)x);
+  const unsigned v = (unsigned)(x < 0 ? -x : x);
   int e = 0;
   while ((v >> (e + 1)) != 0) ++e;
   const unsigned mant = (v << (10 - e)) & 0x3ffu;
   return (uint16_t)(sign | ((unsigned)(e + 15) << 10) | mant);
 }
+struct F16Codes {
+  uint16_t bits[256] = {};
+  constexpr F16Codes() {
+    for (int i = 0; i < 256; ++i) bits[i] = f16_bits(i - 128);
+  }
+};
+constexpr F16Codes kF16Codes;
+// Binding converts every weight up to twice; a table lookup each keeps that
+// behind the copies (4 layers of H 256: 28.4 ms by computing the bits).
+inline uint16_t int8_to_f16_bits(int8_t x) { return kF16Codes.bits[x + 128]; }
 
 struct DevLayer {
   uint16_t* w_qkv = nullptr;
@@ -159,9 +169,10 @@ struct EosHipEncoder {
     size_t o = 0;
     for (int nt = 0; nt < n / 32; ++nt)
       for (int ks = 0; ks < k / 16; ++ks)
-        for (int lane = 0; lane < 64; ++lane)
-          for (int e = 0; e < 8; ++e)
-            f[o++] = int8_to_f16_bits(src[(size_t)(32 * nt + (lane & 31)) * k + 16 * ks + 8 * (lane >> 5) + e]);
+        for (int lane = 0; lane < 64; ++lane) {
+          const int8_t* row = src + (size_t)(32 * nt + (lane & 31)) * k + 16 * ks + 8 * (lane >> 5);
+          for (int e = 0; e < 8; ++e) f[o++] = int8_to_f16_bits(row[e]);
+        }
     return upload(dst, f.data(), f.size(), err);
   }
   int upload_frag8(int8_t** dst, const int8_t* src, int n, int k, char** err) {
@@ -169,9 +180,8 @@ struct EosHipEncoder {
     size_t o = 0;
     for (int nt = 0; nt < n / 32; ++nt)
       for (int ks = 0; ks < k / 32; ++ks)
-        for (int lane = 0; lane < 64; ++lane)
-          for (int e = 0; e < 16; ++e)
-            f[o++] = src[(size_t)(32 * nt + (lane & 31)) * k + 32 * ks + 16 * (lane >> 5) + e];
+        for (int lane = 0; lane < 64; ++lane, o += 16)
+          memcpy(&f[o], src + (size_t)(32 * nt + (lane & 31)) * k + 32 * ks + 16 * (lane >> 5), 16);
     return upload(dst, f.data(), f.size(), err);
   }
 
