@@ -218,14 +218,17 @@ struct EosHipEncoder {
   //    which the wide GEMM after a LayerNorm launch does not: H 384 2,048
   //    rows 226 against 258, 4,096 307 / 289; H 768 1,024 311 / 301, 2,048
   //    424 / 359; H 256 8,192 283 / 300; H 128 32,768 385 / 404.
-  //  - the fused tail (H 384, 512) above kTailRows. One row block takes it as
+  //  - the fused tail (H 384, 512) above tail_rows(). One row block takes it as
   //    long as one on every CU: H 384 4,096 rows 289 against 356, 8,192 390 /
-  //    396, 32,768 1042 / 860; H 512 4,096 353 / 411, 8,192 473 / 460. At H 768
+  //    396, 32,768 1042 / 860; H 512 4,096 353 / 411, 8,192 473 / 460. With F
+  //    of 2 H and less a block is through its weights sooner (3 layers, F = H:
+  //    H 384 5,120 rows 206 / 217, 6,144 238 / 221; H 512 4,096 214 / 232, 6,144
+  //    254 / 252, 7,680 276 / 258). At H 768
   //    a 32-row block carries all 8 MB of weights and the GEMMs win at every
   //    size (8,192 rows 792 against 833, 32,768 2499 / 3133).
   //  - LayerNorm, GEMM launches otherwise (and lin16 for O and FFN down while
   //    their tiles are few, below).
-  static constexpr int kTailRows = 7680;
+  int tail_rows() const { return desc.intermediate > 2 * desc.hidden ? 7680 : 5632; }
   size_t lin_rows() const { return (size_t)550000000 / ((size_t)desc.hidden * desc.hidden); }
 
   int ensure_activations(int batch, int tokens, char** err) {
@@ -456,7 +459,7 @@ struct EosHipEncoder {
                         "enc_ln");
     };
     const bool wide_tail = a8 && fused_tail && (H == 384 || H == 512) && F <= 4 * H &&
-                           max_rows > kTailRows;
+                           max_rows > tail_rows();
     const bool small = a8 && fused_tail && !wide_tail && (size_t)max_rows <= lin_rows();
     // Fused tail: the largest row block whose LDS fits the hidden width.
     const char* tail_name = nullptr;

@@ -62,3 +62,42 @@ def test_small_and_large_batches_agree_bit_for_bit(rt, hidden, heads, batch):
         n = int(mask[b].sum())
         np.testing.assert_array_equal(enc.embed(ids[b:b + 1, :n], mask[b:b + 1, :n])[0], large[b])
     enc.release()
+
+
+@pytest.mark.parametrize("hidden,heads,inter,gelu,batch,least", [
+    (384, 12, 1536, 1, 40, 1),
+    (384, 6, 384, 2, 30, 1),      # the tail from fewer rows on at F <= 2 H
+    (384, 12, 1536, 2, 64, 150),
+    (512, 8, 1024, 1, 30, 1),
+    (512, 8, 2048, 2, 110, 150),  # rows past one 64-row block per CU: the 32-row launch
+])
+def test_large_batches_take_the_fused_tail(rt, hidden, heads, inter, gelu, batch, least):
+    """Batches of more than 7,680 packed rows (5,632 at F <= 2 H) run the fused
+    layer tail at hidden 384 and 512 (a single sequence does not): bit-identical
+    to the unfused launches, and within the contract of the CPU oracle."""
+    from eos_amd.encoder import Encoder
+    print(f"[case] fused tail H={hidden} F={inter} gelu={gelu} batch={batch}", flush=True)
+    w = datagen.bert_q8_weights(2, hidden, heads, inter, 500, 250, seed=hidden + batch, gelu=gelu,
+                                random_affine=True)
+    ids, mask, _ = datagen.encoder_batch(batch, 200, 500, least, 200, 17, 18)
+    enc = Encoder(rt, w)
+    enc.embed(ids[:1], mask[:1])
+    rt.profile(True)
+    rt.profile_reset()
+    got = enc.embed(ids, mask)
+    assert rt.profile_read("enc_tail")[0] >= 2
+    rt.profile_reset()
+    enc.embed(ids[:1], mask[:1])
+    assert rt.profile_read("enc_tail")[0] == 0
+    rt.profile(False)
+    enc.set_fused_tail(False)
+    np.testing.assert_array_equal(got, enc.embed(ids, mask))
+    if gelu == 1:  # the oracle's GELU
+        for b in (0, batch // 2, batch - 1):
+            n = int(mask[b].sum())
+            want = oracle.bert_embed(w.tok, w.pos, w.typ, w.emb_gamma, w.emb_beta,
+                                     [L.dequantized() for L in w.layers], ids[b:b + 1, :n],
+                                     mask[b:b + 1, :n], None, heads, w.ln_eps)
+            cos = (got[b] @ want[0]) / np.linalg.norm(got[b]) / np.linalg.norm(want[0])
+            assert cos >= 0.9999 and np.abs(got[b] - want[0]).max() <= 2e-2
+    enc.release()
