@@ -16,9 +16,8 @@ CPU pins of the oracle:
   outside it;
 - encode -> scan: scores estimate the true inner products within the
   quantization noise, and a vector's own score is its best one.
-GPU: codes and norms are bit-exact against the oracle (both kernels: d <= 512
-and d <= 1024), including zero rows, ragged counts and odd row widths; host and
-device entry points agree; encoder output -> encode on the device matches."""
+GPU: codes and norms are bit-exact against the oracle, including zero rows,
+ragged counts and odd row widths; host and device entry points agree; encoder output -> encode on the device matches."""
 import math
 
 import numpy as np

@@ -1,8 +1,9 @@
-"""The inner-product encode on the f64 matrix cores (eos_tq_encode_ip_s*, _t*):
-codes, signs, ResNorm and Norm bit-exact against the CPU oracle at the edges
-of its tiles (16 rows and vectors, 128 coordinates per kernel variant, 32 or
-16 vectors per workgroup, 64-wide K chunks), with zero, infinite and NaN
-vectors and exact ties."""
+"""The inner-product encode on the f64 matrix cores: codes, signs, ResNorm and
+Norm bit-exact against the CPU oracle at the edges of its tiles (16 rows and
+vectors, 128 coordinates per kernel variant, 64-wide K chunks), with zero,
+infinite and NaN vectors and exact ties. Calls of up to 16 vectors a CU run
+eos_tq_encode_ip_s* (16 vectors per workgroup), larger ones eos_tq_encode_ip_t*
+(32, above dim 512 16)."""
 import numpy as np
 import pytest
 
@@ -62,3 +63,37 @@ def test_encode_ip_large_calls_equal_small_ones(rt, d, bits):
     parts = [qz.encode(x[i:i + 1111]) for i in range(0, n, 1111)]
     for w, *p in zip(whole, *parts):
         np.testing.assert_array_equal(w, np.concatenate(p))
+
+
+@pytest.mark.parametrize("d,bits,rotate", [(96, 3, False), (200, 3, True), (384, 3, True),
+                                           (512, 2, False), (640, 4, True), (768, 3, True),
+                                           (800, 2, True), (1024, 1, False)])
+def test_encode_ip_large_calls_match_oracle(rt, d, bits, rotate):
+    """eos_tq_encode_ip_t* of every width: zero, infinite, NaN and one-hot
+    vectors in the first and in the last, partial workgroup against the
+    oracle, all others against the same vectors in small calls."""
+    n = 16 * rt.info()["compute_units"] + 41
+    print(f"[case] ip encode large against oracle d={d} bits={bits} n={n}", flush=True)
+    rng = np.random.default_rng(d + 7 * bits)
+    rot = np.linalg.qr(rng.normal(size=(d, d)))[0].astype(np.float32) if rotate else None
+    S = rng.normal(size=(d, d)).astype(np.float32)
+    cb = np.linspace(-127, 127, 1 << bits).round().astype(np.int8)
+    s_c = float(np.float32(2.5 / np.sqrt(d) / 127))
+    x = rng.normal(size=(n, d)).astype(np.float32)
+    for i in (0, n - 9):
+        x[i:i + 2] = 0
+        x[i + 1, d // 2] = 2.0
+        x[i + 2, 0] = np.inf
+        x[i + 3, d - 1] = np.nan
+        x[i + 4] *= np.float32(1e-30)
+        x[i + 5] *= np.float32(1e30)
+    iq = IPQuantizer(rt, d, bits, cb, s_c, rot, S)
+    edge = np.r_[0:34, n - 43:n]
+    with np.errstate(all="ignore"):
+        whole = iq.encode(x)
+        want = oracle.tq_encode_ip(x[edge], rot, S, d, bits, cb, s_c)
+        parts = [iq.encode(x[i:i + 1000]) for i in range(0, n, 1000)]
+    for w, o, *p in zip(whole, want, *parts):
+        np.testing.assert_array_equal(w[edge], o)
+        np.testing.assert_array_equal(w, np.concatenate(p))
+    iq.release()
