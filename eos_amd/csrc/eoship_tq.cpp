@@ -236,9 +236,13 @@ struct EosHipTQ {
   // + |R_j| 33 * 2^-23     (32 products of a chunk summed in f32, an ulp lost
   //                         at each addition whatever the order)
   // + |R_j| chunks * 2^-24 (the sum over the chunks)
-  // with 5 % on top for the second-order terms (d = 384: 1.1e-5). Scales that
-  // would put the distance over a quarter of a half step, or leave f32 and
-  // bf16 no room, keep the f64 kernels (rot_frag stays NULL).
+  // with 5 % on top for the second-order terms (d = 384: 1.1e-5). How the MFMA
+  // adds inside a chunk is not documented; an ulp of the running sum per
+  // addition is assumed. Measured with rows and vectors whose every dropped
+  // part and rounding has one sign, next to decision points, d 32 to 768: at most
+  // 3.3e-6, a quarter of the bound.
+  // Scales that would put the distance over a quarter of a half step, or leave
+  // f32 and bf16 no room, keep the f64 kernels (rot_frag stays NULL).
   // R is uploaded once; its transpose and the sums come from the device. Two
   // uploads and passes over d^2 values on the host were most of binding a small
   // corpus (no vectors: d = 384 1.06 ms, d = 1024 7.1, now 0.12 and 0.24).
@@ -2150,11 +2154,16 @@ int eoship_tq_ip_encode_device(EosHipRuntime* rt, const EosHipTQIPSpec* spec, co
   a.n = n;
   // 128 coordinates per tile row of the kernel (TJ); 32 vectors per workgroup
   // while their residuals fit the LDS beside the stages (d <= 512), else 16.
-  // Up to 16 vectors a CU a workgroup's own latency is the call: half the
-  // vectors and twice the load depth (us at n = 273: dim 150 35 -> 24, and
-  // n = 4,096: dim 384 62, where 6,000 in workgroups of 32 takes 100).
-  const bool small = n <= 16 * (int64_t)rt->compute_units;
-  const int tj = (a.d + 127) / 128, per = tj <= 4 && !small ? 32 : 16;
+  // At d <= 512, up to 16 vectors a CU, a workgroup's own latency is the call:
+  // half the vectors and twice the load depth (us, 32 vectors / 16: d = 256
+  // 53 / 35, d = 384 101 / 65, d = 512 170 / 104 at any n up to 4,096). From
+  // 4,097 on the smaller workgroups share CUs (d = 384: 4,097 106 / 126, 8,192
+  // 112 / 132, 65,536 805 / 962; where 32 vectors just begin a second round
+  // they would win again, 8,193 206 / 185). Above d = 512 both take 16 vectors
+  // and the deeper loads only cost registers (d = 768: 205 / 222).
+  const int tj = (a.d + 127) / 128;
+  const bool small = tj <= 4 && n <= 16 * (int64_t)rt->compute_units;
+  const int per = tj <= 4 && !small ? 32 : 16;
   char name[32];
   snprintf(name, sizeof(name), "eos_tq_encode_ip_%c%d", small ? 's' : 't', tj);
   return rt->launch(name, dim3((unsigned)((n + per - 1) / per)), dim3(512), 0, &a, err,

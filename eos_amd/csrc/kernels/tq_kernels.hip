@@ -478,7 +478,7 @@ extern "C" __global__ __launch_bounds__(256) void eos_tq_encode_d1024(TqEncodeAr
 // estimator (the quantizer is in the un-vendored module; byte layout of
 // runtime/turboquant_bytes.go:14-25): the MSE stage of encode_body, then a
 // 1-bit QJL sketch of the residual in the rotated frame, all in f64
-// (encoded by eos_tq_encode_ip_t*):
+// (encoded by eos_tq_encode_ip_s* and _t*):
 //   r_j = u_j - nrm c_code_j;  ResNorm = (float)(sqrt(sum_j r_j^2) / nrm)
 //   sign bit i = (sum_j S[i][j] r_j >= 0), fma chains in j order
 constexpr int kIpDMax = 1024;

@@ -691,7 +691,7 @@ namespace {
 // wavefronts per SIMD).
 // P: steps (of four K values) a fragment load brings. Up to 16 vectors a CU
 // nothing hides a load's latency but the chain itself, so those calls take NV
-// = 1 and P = 8 (see the dispatch for both sides).
+// = 1 and P = 8 at d <= 512 (see the dispatch for both sides).
 template <int NV, int TJ, int P>
 struct EncodeIp {
   static constexpr int BV = 16 * NV, KC = 64, XST = KC + 4, RST = 128 * TJ + 4;
@@ -947,8 +947,4 @@ EOS_TQ_ENCODE_IP(s, 1, 1, 8)
 EOS_TQ_ENCODE_IP(s, 1, 2, 8)
 EOS_TQ_ENCODE_IP(s, 1, 3, 8)
 EOS_TQ_ENCODE_IP(s, 1, 4, 8)
-EOS_TQ_ENCODE_IP(s, 1, 5, 8)
-EOS_TQ_ENCODE_IP(s, 1, 6, 8)
-EOS_TQ_ENCODE_IP(s, 1, 7, 8)
-EOS_TQ_ENCODE_IP(s, 1, 8, 8)
 #undef EOS_TQ_ENCODE_IP

@@ -1,9 +1,9 @@
 """The inner-product encode on the f64 matrix cores: codes, signs, ResNorm and
 Norm bit-exact against the CPU oracle at the edges of its tiles (16 rows and
 vectors, 128 coordinates per kernel variant, 64-wide K chunks), with zero,
-infinite and NaN vectors and exact ties. Calls of up to 16 vectors a CU run
-eos_tq_encode_ip_s* (16 vectors per workgroup), larger ones eos_tq_encode_ip_t*
-(32, above dim 512 16)."""
+infinite and NaN vectors and exact ties. Calls of up to 16 vectors a CU and
+dims up to 512 run eos_tq_encode_ip_s* (16 vectors per workgroup), others
+eos_tq_encode_ip_t* (32, above dim 512 16)."""
 import numpy as np
 import pytest
 
