@@ -152,8 +152,8 @@ struct TqParentArgs {
   long long np, stride;
   double penalty;
   int top_n, qb;
-  // eos_tq_parent_agg: the parents it takes (np of them; p = list[i]), out
-  // rows out_stride apart; NULL: parent p = i.
+  // eos_tq_parent_agg: the parents it takes (np of them, each with children;
+  // p = list[i]), out rows out_stride apart.
   const long long* list;
   long long out_stride;
 };

@@ -2604,8 +2604,9 @@ EOS_DEV void tq_maxsim_body(const TqMaxsimArgs& a) {
 // The bound filter over 8 query groups a pass. At 12.8 million rows of dim
 // 128 x 32 queries of 32 tokens: 2360 us with four vector instructions an
 // element, 2076 with maxsim_bound_short, 1765 with 8 groups a pass and a list
-// per group; the vector unit is busy 71 % of it (327 instructions a tile, 192
-// of them the bound), the matrix unit 51 %, at 1.8 GHz.
+// per group (the vector unit busy 71 % of it, 327 instructions a tile, 192 of
+// them the bound; the matrix unit 51 %, at 1.8 GHz), 1720 with the lists
+// appended in batches.
 #define EOS_TQ_MAXSIM_WIDE(BITS, KS)                                                        \
   extern "C" __global__ __launch_bounds__(kScanThreads) __attribute__((amdgpu_waves_per_eu(3))) \
   void eos_tq_maxsim_b##BITS##_k##KS##_g8_h(TqMaxsimArgs a) {                                \
@@ -2661,7 +2662,7 @@ EOS_TQ_MAXSIM(4, 32, 1)
 
 // ------------------------------------------------------- parent aggregation
 
-// One wavefront per (query, parent): each lane keeps the 5 best of the child
+// One wavefront per (query, listed parent): each lane keeps the 5 best of the child
 // scores it reads (sorted descending in registers, 8 loads in flight), then
 // the wave pops the best min(top_n, count) values in descending order --
 // the order aggregateMultiVectorParentScores sums the accumulator's list in
@@ -2673,14 +2674,10 @@ extern "C" __global__ __launch_bounds__(256) void eos_tq_parent_agg(TqParentArgs
   const long long i = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int q = blockIdx.y;
   if (i >= a.np || q >= a.qb) return;
-  const long long p = a.list != nullptr ? a.list[i] : i;
+  const long long p = a.list[i];
   const long long c0 = a.off[p], c1 = a.off[p + 1];
   const long long cnt = c1 - c0;
   float* out = a.out + (size_t)q * a.out_stride + p;
-  if (cnt <= 0) {
-    if (lane == 0) *out = -__builtin_inff();
-    return;
-  }
   const float* row = a.scores + (size_t)q * a.stride;
   float t[5];
 #pragma unroll
@@ -2731,7 +2728,7 @@ extern "C" __global__ __launch_bounds__(256) void eos_tq_parent_agg(TqParentArgs
 // The same for parents of at most EOS_PARENT_SHORT children, one lane per (query,
 // parent): a wavefront per parent leaves most of its lanes idle there and
 // pays a wavefront's launch, ballots and shuffles for a handful of loads
-// (40,000 parents of 1..13 children, 16 queries: 237 us; this kernel 6 us,
+// (40,000 parents of 1..13 children, 16 queries: 237 us; this kernel 11 us,
 // bound by the latency of a lane's loads, 8 of which are in flight). Longer
 // parents are skipped; the host lists them for eos_tq_parent_agg. The lane
 // keeps the same 5 best and adds them in the same descending order.
