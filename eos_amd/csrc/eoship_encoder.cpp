@@ -44,7 +44,7 @@ constexpr F16Codes kF16Codes;
 inline uint16_t int8_to_f16_bits(int8_t x) { return kF16Codes.bits[x + 128]; }
 
 struct DevLayer {
-  uint16_t* w_qkv = nullptr;
+  uint16_t* w_qkv = nullptr;  // f16 codes (compact family only, as w_1)
   float* s_qkv = nullptr;
   float* b_qkv = nullptr;
   uint16_t* w_o = nullptr;
@@ -697,14 +697,13 @@ int eoship_encoder_bind(EosHipRuntime* rt, const EosHipEncoderDesc* desc, const 
         return fail();
       }
     DevLayer d;
-    if (enc->upload_codes(&d.w_qkv, s.w_qkv, (size_t)3 * H * H, err) ||
-        enc->upload(&d.s_qkv, s.s_qkv, (size_t)3 * H, err) ||
+    // QKV and FFN up run on int8 codes only: no f16 copies.
+    if (enc->upload(&d.s_qkv, s.s_qkv, (size_t)3 * H, err) ||
         enc->upload(&d.b_qkv, s.b_qkv, (size_t)3 * H, err) ||
         enc->upload_codes(&d.w_o, s.w_o, (size_t)H * H, err) ||
         enc->upload(&d.s_o, s.s_o, (size_t)H, err) || enc->upload(&d.b_o, s.b_o, (size_t)H, err) ||
         enc->upload(&d.g1, s.ln1_gamma, (size_t)H, err) ||
         enc->upload(&d.be1, s.ln1_beta, (size_t)H, err) ||
-        enc->upload_codes(&d.w_1, s.w_1, (size_t)F * H, err) ||
         enc->upload(&d.s_1, s.s_1, (size_t)F, err) || enc->upload(&d.b_1, s.b_1, (size_t)F, err) ||
         enc->upload_codes(&d.w_2, s.w_2, (size_t)H * F, err) ||
         enc->upload(&d.s_2, s.s_2, (size_t)H, err) || enc->upload(&d.b_2, s.b_2, (size_t)H, err) ||
