@@ -2604,9 +2604,9 @@ EOS_DEV void tq_maxsim_body(const TqMaxsimArgs& a) {
 // The bound filter over 8 query groups a pass. At 12.8 million rows of dim
 // 128 x 32 queries of 32 tokens: 2360 us with four vector instructions an
 // element, 2076 with maxsim_bound_short, 1765 with 8 groups a pass and a list
-// per group (the vector unit busy 71 % of it, 327 instructions a tile, 192 of
-// them the bound; the matrix unit 51 %, at 1.8 GHz), 1720 with the lists
-// appended in batches.
+// per group, 1720 with the lists appended in batches (359 vector instructions a
+// tile, 192 of them the bound, beside 32 MFMAs; at 1.8 GHz the vector unit is
+// about two thirds busy, the matrix unit half).
 #define EOS_TQ_MAXSIM_WIDE(BITS, KS)                                                        \
   extern "C" __global__ __launch_bounds__(kScanThreads) __attribute__((amdgpu_waves_per_eu(3))) \
   void eos_tq_maxsim_b##BITS##_k##KS##_g8_h(TqMaxsimArgs a) {                                \
