@@ -279,10 +279,11 @@ def test_w8a8_outlier_channels(rt):
 @pytest.mark.parametrize("hidden,heads,inter,gelu", [(384, 12, 1536, 1), (384, 6, 768, 2),
                                                       (512, 8, 2048, 1), (768, 12, 3072, 1)])
 def test_fused_tail_matches_unfused_and_oracle(rt, hidden, heads, inter, gelu):
-    """The fused layer tail (O projection through the second LayerNorm in one
-    kernel per row block) against the unfused GEMM + LayerNorm launches, which
-    round at the same points: embeddings equal to within a few f16 units, and
-    both within the contract against the oracle. Ragged lengths put partial
+    """The fused layer path of a batch of 1,863 packed rows (linear layers with
+    the LayerNorms inside; the tail kernels, which larger batches take, are in
+    test_encoder_small_gpu.py) against the unfused GEMM + LayerNorm launches,
+    which round at the same points: embeddings equal to within a few f16 units,
+    and both within the contract against the oracle. Ragged lengths put partial
     row blocks at every sequence boundary and at the end."""
     _case(f"fused tail H={hidden} heads={heads} F={inter} gelu={gelu}")
     w = datagen.bert_q8_weights(2, hidden, heads, inter, 3000, 256, seed=hidden + gelu,

@@ -3,7 +3,8 @@ bit-identical to the unfused launches at the edges of their tiles (32 and 64
 rows, 256 and 128 columns) for every width, both GELUs, both poolings and
 token types, and within the contract of the CPU oracle; and bit-identical to
 the same sequence in batches that take the other paths (LayerNorm launches
-with the wide GEMM, 64-row tiles, the fused tail)."""
+with the wide GEMM, 64-row tiles, the fused tail); and batches above the
+tail's line by the tail kernels."""
 import numpy as np
 import pytest
 

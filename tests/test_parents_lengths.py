@@ -19,7 +19,7 @@ def _offsets(counts):
     ("all long", [65] * 40, 7),
     ("all short", [1, 2, 3, 4, 5, 6] * 50, 300),
     ("mixed, chunked ranking", [1, 3, 0, 5, 2, 70, 4, 1] * 2500, 50),
-    ("chunked ranking, k near a chunk", [1, 2] * 5000, 1000),
+    ("a tenth of the parents", [1, 2] * 5000, 1000),
 ])
 def test_parent_lengths_match_oracle(rt, name, counts, k):
     from eos_amd.turboquant import TurboQuantIndex, TurboQuantParents
