@@ -280,7 +280,8 @@ def test_w8a8_outlier_channels(rt):
                                                       (512, 8, 2048, 1), (768, 12, 3072, 1)])
 def test_fused_tail_matches_unfused_and_oracle(rt, hidden, heads, inter, gelu):
     """The fused layer path of a batch of 1,863 packed rows (linear layers with
-    the LayerNorms inside; the tail kernels, which larger batches take, are in
+    the LayerNorms inside, at hidden 768 the small projections beside GEMM and
+    LayerNorm launches; the tail kernels, which larger batches take, are in
     test_encoder_small_gpu.py) against the unfused GEMM + LayerNorm launches,
     which round at the same points: embeddings equal to within a few f16 units,
     and both within the contract against the oracle. Ragged lengths put partial
